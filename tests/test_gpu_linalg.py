@@ -280,3 +280,26 @@ def test_autotuned_ctm_matches_oracle():
     assert abs(gE - E) < 1e-10 * abs(E), (gE, E)
     del genv
     ctx.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 15, 16, 17, 31, 48, 100, 112, 113, 127, 128])
+@pytest.mark.parametrize("deficient", [False, True])
+def test_tall_svd_block_edges(gpu_ctx, p, deficient):
+    """CholeskyQR of a tall block at the 16-wide block edges of its
+    factorisation: singular values, left basis and reconstruction against
+    LAPACK; with a zero and a dependent column the range is kept and the
+    dropped directions carry no weight.  Columns of lengths over six decades.
+    Tolerance: three passes leave ||Q^T Q - 1|| at a few p eps = 128 * 2.2e-16,
+    times ten for the products around them: 3e-13 of the largest value."""
+    rng = np.random.default_rng(100 + p)
+    A = rng.standard_normal((300, p)) * np.logspace(0, -6, p)
+    if deficient and p >= 3:
+        A[:, p // 2] = 0.0
+        A[:, p - 1] = 2.0 * A[:, 0]
+    U, s, V = ta.svd_top(gpu_ctx.tensor(A), p)
+    U, V = U.numpy(), V.numpy()
+    ref = np.linalg.svd(A, compute_uv=False)
+    assert np.max(np.abs(s - ref)) < 3e-13 * ref[0]
+    assert np.max(np.abs((U * s) @ V.T - A)) < 3e-13 * ref[0]
+    r = p - 2 if deficient and p >= 3 else p
+    assert np.max(np.abs(U[:, :r].T @ U[:, :r] - np.eye(r))) < 3e-13
