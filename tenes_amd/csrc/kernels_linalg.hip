@@ -15,6 +15,8 @@
 //                       without keeping a second p x p matrix in LDS.
 //  * sort_desc        : rank sort of singular values, descending.
 #include <cfloat>
+#include <type_traits>
+#include <utility>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -87,19 +89,30 @@ __global__ void refill_columns_kernel(double *X, int64_t n, int p,
 
 // ---------------------------------------------------------------------------
 // Shifted Cholesky + inverse of the upper factor: blocked, one workgroup of
-// 4 waves, the padded matrix resident in LDS, diagonally scaled first.
+// 8 waves, the padded matrix resident in LDS, diagonally scaled first.
 //
-// Blocks of 16.  Per block column: wave 0 factors the 16 x 16 diagonal block
-// (lane l / register t holds element (l/16 + 4t, l%16); the pivot row is
-// broadcast through a 16-entry LDS row, wave-synchronous, no barrier), the
-// block row of R is a forward substitution with one thread per column, and
-// the trailing update runs on the FP64 MFMA.  After the sweep the diagonal
-// blocks are inverted in parallel (one 16-lane group per block) and the
-// off-diagonal blocks of R^{-1} follow by block back substitution on the
-// MFMA, whose output registers are directly the B operand of the next
-// product.  Barriers: 3 per block column + 1 per block row of the inverse.
+// One CU and a chain of p dependent pivots bound it, so everything that is
+// not on that chain runs beside it.  Blocks of 16.  The 16 x 16 diagonal
+// block is factored by one wave with column lc in lane lc of each 16-lane row
+// (the four rows do the same work), an element of another column coming by
+// DPP row_newbcast: a pivot step is a broadcast, a reciprocal square root and
+// one multiply before the next pivot is known.  Per block column kb, two
+// phases:
+//   A  block row of F (forward substitution, one thread per column, the
+//      diagonal block's entries again by DPP) and, on another wave, the
+//      inverse of the diagonal block;
+//   B  wave 0 updates the next diagonal block and factors it while the other
+//      waves do the rest of the trailing update on the FP64 MFMA.
+// Alone on the device, average over a projector's calls at 128 x 128: 93 us
+// before (4 waves, pivots through LDS with a division each, substitutions
+// through LDS broadcasts, the inverse after the factor), 39 us now; 8 x 8:
+// 14.8 us before, 5.6 us now.
 // ---------------------------------------------------------------------------
-constexpr int kCholThreads = 256;
+constexpr int kCholThreads = 512;
+constexpr int kCholWaves = kCholThreads / 64;
+// row length of the LDS matrix: odd against bank conflicts, and one constant
+// for every p so that the offsets are immediates
+constexpr int kCholLd = kMaxDim + 1;
 constexpr int kCholXdLd = 17;  // padded leading dimension of the diagonal inverses
 
 __device__ __forceinline__ d4 mfma16(double a, double b, d4 c) {
@@ -112,51 +125,81 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 }
 
-size_t chol_lds_bytes(int p) {
-  const int pp = (p + 15) / 16 * 16;
-  return ((size_t)pp * (pp + 1) + (size_t)(pp / 16) * 16 * kCholXdLd + 16) *
-         sizeof(double);
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <class F, int... I>
+__device__ __forceinline__ void unroll_impl(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unroll(F f) {
+  unroll_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// v of lane L of the caller's 16-lane row (all lanes of the row active)
+template <int L>
+__device__ __forceinline__ double row_bcast(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + L, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + L, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// 1 / sqrt(x) for positive normal x: the hardware estimate and two Newton
+// steps y += y (1/2 - (x/2) y^2).
+__device__ __forceinline__ double rsqrt_newton(double x) {
+  const double h = 0.5 * x;
+  double y = __builtin_amdgcn_rsq(x);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) y = fma(y, fma(-h * y, y, 0.5), y);
+  return y;
+}
+
+size_t chol_lds_bytes(int p) {
+  const int pp = (p + 15) / 16 * 16;
+  return ((size_t)pp * kCholLd + (size_t)pp * kCholXdLd) * sizeof(double);
+}
+
+// FULL: p == kMaxDim (every pass of the range finder).
+template <bool FULL>
 __global__ __launch_bounds__(kCholThreads) void chol_inv_kernel(
-    const double *G, int p, double shift_coef, double rel_floor, double *R,
+    const double *G, int p_arg, double shift_coef, double rel_floor, double *R,
     double *Rinv, const double *pre) {
   extern __shared__ double lds[];
   __shared__ int defic[kMaxDim];
-  __shared__ double s_dg[kMaxDim], s_scl[kMaxDim];
+  __shared__ double s_diag[kMaxDim], s_dg[kMaxDim], s_scl[kMaxDim];
   __shared__ double s_rd[kMaxDim];  // 1 / F[i][i] (0 for a dropped column)
   __shared__ double s_shift, s_thr, s_floor;
   __shared__ int s_zero, s_near;
+  const int p = FULL ? kMaxDim : p_arg;
   const int pp = (p + 15) / 16 * 16;  // padded size (identity padding)
   const int nb = pp / 16;
-  const int ld = pp + 1;
-  double *A = lds;                     // pp x ld, upper triangle: G, then F
+  constexpr int ld = kCholLd;
+  // A: pp x ld, the upper triangle of 16 x 16 blocks holds G, then F; below
+  // it block (bj, bi) holds the transpose of X's block (bi, bj), bi < bj
+  double *A = lds;
   double *Xd = lds + (size_t)pp * ld;  // nb blocks of 16 x kCholXdLd: F_kk^-1
-  double *rowbuf = Xd + (size_t)nb * 16 * kCholXdLd;  // 16: pivot row
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
+  // the wave's number as a scalar: its branches are uniform
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane >> 4, lc = lane & 15;  // (row in 4-group, column)
-  const int c0 = tid & 63, r0 = tid >> 6;    // load/store mapping
+  const int c0 = lane, r0 = w;               // load/store mapping
 
-  // Load: thread -> columns c0, c0 + 64 and rows r0 + 4u; all 64 loads of a
-  // thread are issued before the first LDS store (one memory round trip).
-  {
-    double v[32][2];
+  // Load: thread -> columns c0, c0 + 64 and rows r0 + 8u.  The full size
+  // holds its 32 values in registers (all loads in flight together) until the
+  // scales are known; smaller ones go through LDS.
+  double v[FULL ? 16 : 1][2];
+  if (tid == 0) s_near = 1;
+  if constexpr (FULL) {
 #pragma unroll
-    for (int u = 0; u < 32; ++u)
+    for (int u = 0; u < 16; ++u)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = r0 + 4 * u, c = c0 + 64 * h;
-        const bool in = r < p && c < p;
-        const double g = G[in ? r * p + c : 0];
-        v[u][h] = in ? g : (r == c ? 1.0 : 0.0);
-      }
-#pragma unroll
-    for (int u = 0; u < 32; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = r0 + 4 * u, c = c0 + 64 * h;
-        if (r < pp && c < pp) A[r * ld + c] = v[u][h];
+      for (int h = 0; h < 2; ++h) v[u][h] = G[(r0 + 8 * u) * kMaxDim + c0 + 64 * h];
+    if (tid < kMaxDim) s_diag[tid] = G[tid * (kMaxDim + 1)];
+  } else {
+    for (int r = r0; r < pp; r += kCholWaves)
+      for (int c = c0; c < pp; c += 64) {
+        const double g = r < p && c < p ? G[r * p + c] : (r == c ? 1.0 : 0.0);
+        A[r * ld + c] = g;
+        if (r == c) s_diag[r] = g;
       }
   }
   __syncthreads();
@@ -167,27 +210,40 @@ __global__ __launch_bounds__(kCholThreads) void chol_inv_kernel(
   // one); zero columns keep a zero diagonal.
   // A pre-scaled input (pre != nullptr: a diagonal block or Schur
   // complement of a larger scaled and shifted Gram matrix) keeps unit scales.
-  for (int i = tid; i < pp; i += kCholThreads) {
-    const double g = A[i * ld + i];
-    const double dg = (i < p && !pre) ? (g > 0.0 ? sqrt(g) : 0.0) : 1.0;
-    s_dg[i] = dg;
-    s_scl[i] = dg > 0.0 ? 1.0 / dg : 0.0;
+  if (tid < pp) {
+    const double g = s_diag[tid];
+    const double dg = (tid < p && !pre) ? (g > 0.0 ? sqrt(g) : 0.0) : 1.0;
+    s_dg[tid] = dg;
+    s_scl[tid] = dg > 0.0 ? 1.0 / dg : 0.0;
   }
   __syncthreads();
-  if (!pre) {
-#pragma unroll 4
-    for (int u = 0; u < 32; ++u)
+  {
+    bool near = true;
+    if constexpr (FULL) {
+      const double sc[2] = {s_scl[c0], s_scl[c0 + 64]};
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = r0 + 4 * u, c = c0 + 64 * h;
-        if (r < pp && c < pp) A[r * ld + c] = (A[r * ld + c] * s_scl[r]) * s_scl[c];
-      }
-    __syncthreads();
+      for (int u = 0; u < 16; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int r = r0 + 8 * u, c = c0 + 64 * h;
+          const double g = (v[u][h] * s_scl[r]) * sc[h];
+          A[r * ld + c] = g;
+          near = near && fabs(g - (r == c ? 1.0 : 0.0)) <= 1e-10;
+        }
+    } else {
+      for (int r = r0; r < pp; r += kCholWaves)
+        for (int c = c0; c < pp; c += 64) {
+          const double g = (A[r * ld + c] * s_scl[r]) * s_scl[c];
+          A[r * ld + c] = g;
+          near = near && fabs(g - (r == c ? 1.0 : 0.0)) <= 1e-10;
+        }
+    }
+    if (!near) s_near = 0;
   }
   if (w == 0) {
     double tr = 0.0, mx = 0.0;
     for (int i = lane; i < p; i += 64) {
-      const double g = A[i * ld + i];
+      const double g = (s_diag[i] * s_scl[i]) * s_scl[i];
       tr += fabs(g);
       mx = fmax(mx, g);
     }
@@ -218,7 +274,7 @@ __global__ __launch_bounds__(kCholThreads) void chol_inv_kernel(
   if (s_zero) {
     // Zero (or NaN) Gram matrix: the input block is zero.  R = 0 (the block
     // has no range), Rinv = I so that Q = Y * Rinv stays zero.
-    for (int r = r0; r < p; r += 4)
+    for (int r = r0; r < p; r += kCholWaves)
       for (int c = c0; c < p; c += 64) {
         if (R) R[r * p + c] = 0.0;
         Rinv[r * p + c] = (r == c) ? 1.0 : 0.0;
@@ -231,216 +287,199 @@ __global__ __launch_bounds__(kCholThreads) void chol_inv_kernel(
   // exact to O(||U||^2) <= 2e-16 (||U||_2 <= 128 * 1e-10): no pivot chain.
   // No pivot can fall to the drop threshold (pivots are 1 +- 1e-10), so the
   // factorisation would drop nothing either.
-  if (!pre && shift_coef == 0.0) {
-    if (tid == 0) s_near = 1;
-    __syncthreads();
-    bool near = true;
-#pragma unroll 4
-    for (int u = 0; u < 32; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = r0 + 4 * u, c = c0 + 64 * h;
-        if (r < p && c < p) near = near && fabs(A[r * ld + c] - (r == c ? 1.0 : 0.0)) <= 1e-10;
+  if (!pre && shift_coef == 0.0 && s_near) {
+#pragma unroll 2
+    for (int r = r0; r < p; r += kCholWaves)
+#pragma unroll 2
+      for (int c = c0; c < p; c += 64) {
+        const double e = c > r ? A[r * ld + c] : (c == r ? 0.5 * (A[r * ld + r] - 1.0) : 0.0);
+        const double id = r == c ? 1.0 : 0.0;
+        if (R) R[r * p + c] = (id + e) * s_dg[c];
+        Rinv[r * p + c] = s_scl[r] * (id - e);
       }
-    if (!near) s_near = 0;
-    __syncthreads();
-    if (s_near) {
-#pragma unroll 4
-      for (int u = 0; u < 32; ++u)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int r = r0 + 4 * u, c = c0 + 64 * h;
-          if (r < p && c < p) {
-            const double e = c > r ? A[r * ld + c] : (c == r ? 0.5 * (A[r * ld + r] - 1.0) : 0.0);
-            const double id = r == c ? 1.0 : 0.0;
-            if (R) R[r * p + c] = (id + e) * s_dg[c];
-            Rinv[r * p + c] = s_scl[r] * (id - e);
-          }
-        }
-      return;
-    }
+    return;
   }
-  const double shift = s_shift, thr = s_thr;
-  for (int i = tid; i < p; i += kCholThreads) A[i * ld + i] += shift;
-  __syncthreads();
-  const double floor_d = s_floor;
+  const double shift = s_shift, thr = s_thr, floor_d = s_floor;
+  if (shift != 0.0) {
+    for (int i = tid; i < p; i += kCholThreads) A[i * ld + i] += shift;
+    __syncthreads();
+  }
 
+  // Cholesky of the diagonal block at K0 (one wave): rows of F, reciprocal
+  // pivots and dropped-column flags (unit pivot, zero row) to LDS.
+  auto factor_diag = [&](int K0) {
+    double a[16], rd = 0.0;
+    int drop = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = A[(K0 + r) * ld + K0 + lc];
+    unroll<16>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      double piv = row_bcast<k>(a[k]);
+      const bool dk = thr >= 0.0 && !(piv > thr);
+      if (dk || !(piv > floor_d)) piv = floor_d;
+      const double rs = rsqrt_newton(piv);
+      const double m = dk ? 0.0 : a[k] * rs;
+      unroll<16>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        if constexpr (r > k) a[r] = fma(-row_bcast<r>(m), m, a[r]);
+      });
+      // entries left of the diagonal are meaningless, and never read
+      A[(K0 + k) * ld + K0 + lc] = lc == k ? (dk ? 1.0 : piv * rs) : m;
+      if (lc == k) {
+        rd = dk ? 0.0 : rs;
+        drop = dk ? 1 : 0;
+      }
+    });
+    s_rd[K0 + lc] = rd;
+    defic[K0 + lc] = drop;
+  };
+  // A[I0][J0] -= F[K0][I0]^T F[K0][J0]
+  auto trail = [&](int K0, int I0, int J0) {
+    d4 acc;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = A[(I0 + lr + 4 * q) * ld + J0 + lc];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const double av = -A[(K0 + 4 * s + lr) * ld + I0 + lc];
+      const double bv = A[(K0 + 4 * s + lr) * ld + J0 + lc];
+      acc = mfma16(av, bv, acc);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) A[(I0 + lr + 4 * q) * ld + J0 + lc] = acc[q];
+  };
   for (int kb = 0; kb < nb; ++kb) {
-    const int K0 = kb * 16;
-    // ---- (1) diagonal block: Cholesky, wave 0 --------------------------
-    if (w == 0) {
-      double d[4], pv[4];
-      bool dfc[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        d[t] = A[(K0 + lr + 4 * t) * ld + K0 + lc];
-        pv[t] = 1.0;
-        dfc[t] = false;
-      }
-      // right-looking, rows kept unscaled: D[i][j] -= D[k][i] D[k][j] / d_k
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        if (lr == (k & 3)) rowbuf[lc] = d[k >> 2];  // row k of the block
-        wave_lds_fence();
-        double piv = rowbuf[k];
-        const bool dk = thr >= 0.0 && !(piv > thr);
-        if (!dk && !(piv > floor_d)) piv = floor_d;
-        const double rkc = dk ? 0.0 : rowbuf[lc] / piv;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int r = lr + 4 * t;
-          if (r > k && lc >= r) d[t] -= rowbuf[r] * rkc;
-          if (r == k) {
-            pv[t] = piv;
-            dfc[t] = dk;
-          }
-        }
-        wave_lds_fence();  // all reads of this row before the next store
-      }
-      // F: scaled rows, unit pivot and zero row for dropped columns
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int r = lr + 4 * t;
-        if (lc >= r) {
-          const double sd = sqrt(pv[t]);
-          A[(K0 + r) * ld + K0 + lc] =
-              lc == r ? (dfc[t] ? 1.0 : sd) : (dfc[t] ? 0.0 : d[t] / sd);
-          if (lc == r) s_rd[K0 + r] = dfc[t] ? 0.0 : 1.0 / sd;
-        }
-        if (lc == r) defic[K0 + r] = dfc[t] ? 1 : 0;
-      }
-    }
-    __syncthreads();
-    // ---- (2) block row of F by forward substitution, one thread per column:
-    //   F_kk^T P = A[K0:K0+16, col], rows of dropped columns set to zero.
-    // Column-oriented: once v_t is final (times 1/F[t][t], 0 for a dropped
-    // column) it is eliminated from all later rows at once, so the chain
-    // from one row to the next is one multiply and one FMA (the row-oriented
-    // sums made every row wait for a chain of t FMAs and a division).
-    const int ncol = pp - K0 - 16;
-    if (tid < ncol) {
-      const int col = K0 + 16 + tid;
-      double v[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) v[r] = A[(K0 + r) * ld + col];
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        v[t] *= s_rd[K0 + t];
-#pragma unroll
-        for (int r = t + 1; r < 16; ++r) v[r] -= A[(K0 + t) * ld + K0 + r] * v[t];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) A[(K0 + r) * ld + col] = v[r];
-    }
-    __syncthreads();
-    // ---- (3) trailing update A[bi][bj] -= P[:,bi]^T P[:,bj], bi <= bj ------
+    int K0 = kb * 16;
+    asm volatile("" : "+s"(K0));  // one base address, not one induction variable per row
     const int n = nb - kb - 1;
-    const int nblk = n * (n + 1) / 2;
-    for (int b = w; b < nblk; b += kCholThreads / 64) {
-      int bi = 0, rem = b;
-      while (rem >= n - bi) {  // row-wise enumeration of the upper blocks
-        rem -= n - bi;
-        ++bi;
+    // ---- phase B of block column kb - 1 --------------------------------------
+    if (w == 0) {
+      if (kb > 0) {
+        trail(K0 - 16, K0, K0);
+        wave_lds_fence();
       }
-      const int I0 = (kb + 1 + bi) * 16, J0 = (kb + 1 + bi + rem) * 16;
-      d4 acc;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = A[(I0 + lr + 4 * q) * ld + J0 + lc];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const double av = -A[(K0 + 4 * s + lr) * ld + I0 + lc];
-        const double bv = A[(K0 + 4 * s + lr) * ld + J0 + lc];
-        acc = mfma16(av, bv, acc);
+      factor_diag(K0);
+    } else if (kb > 0) {
+      for (int t = w; t < (n + 1) * (n + 2) / 2; t += kCholWaves - 1) {
+        int bi = 0, rem = t;  // row-wise enumeration of the upper blocks
+        while (rem >= n + 1 - bi) {
+          rem -= n + 1 - bi;
+          ++bi;
+        }
+        trail(K0 - 16, (kb + bi) * 16, (kb + bi + rem) * 16);
       }
+    }
+    __syncthreads();
+    // ---- phase A -----------------------------------------------------------
+    // Block row of F: F_kk^T P = A[K0:K0+16, col], rows of dropped columns
+    // set to zero.  Column-oriented: once v_t is final (times 1/F[t][t], 0
+    // for a dropped column) it is eliminated from all later rows at once.
+    const int ncol = 16 * n;
+    if (w * 64 < ncol) {
+      double x[16];
+      const int col = K0 + 16 + min(tid, ncol - 1);  // idle lanes repeat the last column
+      const double rdv = s_rd[K0 + lc];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) A[(I0 + lr + 4 * q) * ld + J0 + lc] = acc[q];
+      for (int r = 0; r < 16; ++r) x[r] = A[(K0 + r) * ld + col];
+      double f = A[K0 * ld + K0 + lc];  // row t of F_kk, one step ahead
+      unroll<16>([&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        const double fn = A[(K0 + (t < 15 ? t + 1 : t)) * ld + K0 + lc];
+        x[t] *= row_bcast<t>(rdv);
+        unroll<16>([&](auto rc) {
+          constexpr int r = decltype(rc)::value;
+          if constexpr (r > t) x[r] = fma(-row_bcast<r>(f), x[t], x[r]);
+        });
+        f = fn;
+        // without it all 120 broadcasts are hoisted, and spilled
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      // stores without a guard, here and below: the FMAs would be sunk into
+      // the guarded block, away from their broadcasts
+#pragma unroll
+      for (int r = 0; r < 16; ++r) A[(K0 + r) * ld + col] = x[r];
+    } else if (w == kCholWaves - 1) {
+      // F_kk^{-1}, lane lc holding column lc, rows from the bottom:
+      //   X[i][c] = (delta_ic - sum_{k>i} F[i][k] X[k][c]) / F[i][i].
+      // A dropped column i gets a zero row i (and column i) here; no other
+      // column of X depends on it (row i of F is e_i^T, so the exact X[i][c]
+      // is 0 for c != i).
+      double x[16];
+      const double rdv = s_rd[K0 + lc];
+      int id = lc;
+      asm volatile("" : "+v"(id));  // else the unit columns are kept through the loop
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x[r] = id == r ? 1.0 : 0.0;
+      double f = A[(K0 + lc) * ld + K0 + 15];  // column i of F_kk, one step ahead
+      unroll<16>([&](auto tc) {
+        constexpr int i = 15 - decltype(tc)::value;
+        const double fn = A[(K0 + lc) * ld + K0 + (i > 0 ? i - 1 : 0)];
+        x[i] *= row_bcast<i>(rdv);
+        unroll<16>([&](auto rc) {
+          constexpr int r = decltype(rc)::value;
+          if constexpr (r < i) x[r] = fma(-row_bcast<r>(f), x[i], x[r]);
+        });
+        f = fn;
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int r = 0; r < 16; ++r) Xd[(K0 + r) * kCholXdLd + lc] = x[r];
     }
     __syncthreads();
   }
 
-  // ---- diagonal blocks of X = F^{-1}: 16-lane group g of wave w inverts
-  // block 4w + g, lane lc holding column lc, rows from the bottom:
-  //   X[i][c] = (delta_ic - sum_{k>i} F[i][k] X[k][c]) / F[i][i],
-  // column-oriented as the block row above (x_i final, then eliminated from
-  // the rows above it).  A dropped column i gets a zero row i here; its
-  // column of X is zeroed on the store and no other column of X depends on
-  // that row (row i of F is e_i^T, so the exact X[i][c] is 0 for c != i).
+  // ---- X = F^{-1}, block column j on one wave, rows from the bottom:
+  //   X[bi][j] = -F_bi^{-1} sum_{bi<k<=j} F[bi][k] X[k][j],
+  // the sums of all rows in registers, a block's output registers being the
+  // B operand of the next products: no barrier, no LDS round trip.  (Back
+  // substitution by columns keeps F X - I small, which Y X needs; X computed
+  // from X F = I, block column by block column beside the factorisation, lost
+  // the orthogonality of Y X to the condition of F.)  The longest and the
+  // shortest column share a SIMD.  Blocks of X go transposed below the
+  // diagonal.
   {
-    const int b = w * 4 + lr;
-    if (b < nb) {
-      const double *Fb = A + (size_t)b * 16 * ld + b * 16;
-      double x[16];
+    const int j = w < 4 ? nb - 1 - w : w - 4;
+    if (j > 0 && (w < 4 || j < nb - 4)) {
+      d4 T[7], Xc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = lc == i ? 1.0 : 0.0;
+      for (int bi = 0; bi < 7; ++bi) T[bi] = d4{0.0, 0.0, 0.0, 0.0};
+      unroll<7>([&](auto ic) {
+        constexpr int k = 7 - decltype(ic)::value;
+        if (k <= j) {
+          if (k == j) {
 #pragma unroll
-      for (int i = 15; i >= 0; --i) {
-        x[i] *= s_rd[b * 16 + i];
+            for (int s = 0; s < 4; ++s) Xc[s] = Xd[(j * 16 + 4 * s + lr) * kCholXdLd + lc];
+          }
+          unroll<k>([&](auto bc) {
+            constexpr int bi = k - 1 - decltype(bc)::value;
 #pragma unroll
-        for (int r = 0; r < i; ++r) x[r] -= Fb[r * ld + i] * x[i];
-      }
+            for (int s = 0; s < 4; ++s)
+              T[bi] = mfma16(A[(bi * 16 + lc) * ld + k * 16 + 4 * s + lr], Xc[s], T[bi]);
+          });
+          d4 Xo = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int r = 0; r < 16; ++r) Xd[(b * 16 + r) * kCholXdLd + lc] = x[r];
+          for (int s = 0; s < 4; ++s)
+            Xo = mfma16(-Xd[((k - 1) * 16 + lc) * kCholXdLd + 4 * s + lr], T[k - 1][s], Xo);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) A[(j * 16 + lc) * ld + (k - 1) * 16 + lr + 4 * q] = Xo[q];
+          Xc = Xo;
+        }
+      });
     }
   }
   __syncthreads();
 
-  // ---- X = F^{-1}: block back substitution, block rows from the bottom ----
-  // X[bi][bj] = -F_bi^{-1} sum_{bi<k<=bj} F[bi][k] X[k][bj]; off-diagonal
-  // blocks of X are stored transposed in the (unused) lower triangle of A.
-  // The k-sum uses two accumulators to halve the dependent MFMA chain.
-  for (int bi = nb - 2; bi >= 0; --bi) {
-    const int n = nb - 1 - bi;
-    for (int idx = w; idx < n; idx += kCholThreads / 64) {
-      const int bj = bi + 1 + idx;
-      // T += F[bi][k] X[k][bj] for one block k
-      auto accum = [&](d4 T, int k) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int kk = k * 16 + 4 * s + lr;
-          const double av = A[(bi * 16 + lc) * ld + kk];
-          const double bv = (k == bj) ? Xd[(bj * 16 + 4 * s + lr) * kCholXdLd + lc]
-                                      : A[(bj * 16 + lc) * ld + kk];
-          T = mfma16(av, bv, T);
-        }
-        return T;
-      };
-      d4 T0 = {0.0, 0.0, 0.0, 0.0}, T1 = {0.0, 0.0, 0.0, 0.0};
-      int k = bi + 1;
-      for (; k + 1 <= bj; k += 2) {
-        T0 = accum(T0, k);
-        T1 = accum(T1, k + 1);
-      }
-      if (k <= bj) T0 = accum(T0, k);
-      const d4 T = T0 + T1;
-      d4 Xo = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        Xo = mfma16(Xd[(bi * 16 + lc) * kCholXdLd + 4 * s + lr], T[s], Xo);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) A[(bj * 16 + lc) * ld + bi * 16 + lr + 4 * q] = -Xo[q];
-    }
-    __syncthreads();
-  }
-
-#pragma unroll 8
-  for (int u = 0; u < 32; ++u)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int r = r0 + 4 * u, c = c0 + 64 * h;
-      if (r < p && c < p) {
-        double rv = 0.0, xv = 0.0;
-        if (c >= r) {
-          rv = defic[r] ? 0.0 : A[r * ld + c];
-          // a dropped column gets a zero column in R^{-1}: Q = Y R^{-1} then
-          // has an exact zero there instead of an unnormalised residual (the
-          // other columns of Q do not depend on it: row c of F is e_c^T)
-          xv = defic[c] ? 0.0
-                        : ((r >> 4) == (c >> 4) ? Xd[r * kCholXdLd + (c & 15)]
-                                                : A[c * ld + r]);
-        }
-        if (R) R[r * p + c] = rv * s_dg[c];
-        Rinv[r * p + c] = xv * s_scl[r];
-      }
+#pragma unroll 2
+  for (int r = r0; r < p; r += kCholWaves)
+#pragma unroll 2
+    for (int c = c0; c < p; c += 64) {
+      double xv = 0.0;
+      // a dropped column gets a zero column in R^{-1}: Q = Y R^{-1} then
+      // has an exact zero there instead of an unnormalised residual (the
+      // other columns of Q do not depend on it: row c of F is e_c^T)
+      if (c >= r && !defic[c])
+        xv = (r >> 4) == (c >> 4) ? Xd[r * kCholXdLd + (c & 15)] : A[c * ld + r];
+      if (R) R[r * p + c] = (c >= r && !defic[r] ? A[r * ld + c] : 0.0) * s_dg[c];
+      Rinv[r * p + c] = xv * s_scl[r];
     }
 }
 
@@ -962,7 +1001,11 @@ int jacobi_lds_dim() { return kMaxDim; }
 void linalg_init_device() {
   const int lds = kMaxDim * kMaxDim * (int)sizeof(double);
   TN_HIP_CHECK(hipFuncSetAttribute(
-      reinterpret_cast<const void *>(&chol_inv_kernel),
+      reinterpret_cast<const void *>(&chol_inv_kernel<true>),
+      hipFuncAttributeMaxDynamicSharedMemorySize,
+      (int)chol_lds_bytes(kMaxDim)));
+  TN_HIP_CHECK(hipFuncSetAttribute(
+      reinterpret_cast<const void *>(&chol_inv_kernel<false>),
       hipFuncAttributeMaxDynamicSharedMemorySize,
       (int)chol_lds_bytes(kMaxDim)));
   TN_HIP_CHECK(hipFuncSetAttribute(
@@ -1001,8 +1044,12 @@ void chol_inv_upper(const double *G, int p, double shift_coef,
                     const double *pre) {
   TN_REQUIRE(p >= 1 && p <= kMaxDim, "chol_inv_upper: p out of range");
   const size_t lds = chol_lds_bytes(p);
-  hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(kCholThreads), lds, s, G, p,
-                     shift_coef, rel_floor, R, Rinv, pre);
+  if (p == kMaxDim)
+    hipLaunchKernelGGL((chol_inv_kernel<true>), dim3(1), dim3(kCholThreads), lds, s, G, p,
+                       shift_coef, rel_floor, R, Rinv, pre);
+  else
+    hipLaunchKernelGGL((chol_inv_kernel<false>), dim3(1), dim3(kCholThreads), lds, s, G, p,
+                       shift_coef, rel_floor, R, Rinv, pre);
   TN_HIP_CHECK(hipGetLastError());
 }
 
