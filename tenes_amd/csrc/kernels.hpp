@@ -194,9 +194,16 @@ void jacobi_svd(double *W, int m, int p, int batch, double tol,
                 int max_sweeps, double *sigma, double *rot, int *nsteps,
                 hipStream_t s);
 // Rebuild the accumulated rotation matrix J (p x p, row-major) from the
-// rotation stream written by jacobi_svd (batch of 1).
+// rotation stream written by jacobi_svd (batch of 1), or J0 times it (J0, J:
+// rows x p row-major, p <= 128; J0 may be J: a row is read before it is
+// written).
 void jacobi_accumulate(const double *rot, const int *nsteps, int p, double *J,
-                       hipStream_t s);
+                       hipStream_t s, const double *J0 = nullptr, int rows = 0);
+// Preconditioner of jacobi_svd for m, n <= 128 (a batch of m x n row-major
+// matrices): A = W Q^T from the row-pivoted QR of A^T, W (m x r column-major,
+// r = min(m, n)) with columns of falling length, Q (n x r row-major)
+// orthonormal columns, or nullptr.
+void qrp(const double *A, int m, int n, int batch, double *W, double *Q, hipStream_t s);
 // sorted[b][r] = sigma[b][perm[b][r]], descending (ties keep index order).
 void sort_desc(const double *sigma, int p, int batch, double *sorted,
                int *perm, hipStream_t s);

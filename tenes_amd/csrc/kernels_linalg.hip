@@ -643,6 +643,143 @@ __device__ __forceinline__ double sum16(double v) {
   return v;
 }
 
+// Pivoted Householder QR of A^T (A: m x n row-major, m, n <= 128, one
+// workgroup per matrix) as the preconditioner of the one-sided Jacobi SVD:
+//   A = W Q^T, Q (n x r) orthonormal, W = A Q (m x r), r = min(m, n).
+// W is lower triangular up to the order of its rows, with columns of falling
+// length, and its columns are close to orthogonal: the Jacobi needs 5 to 7
+// sweeps on it where the matrices of the small environments (40 x 40, graded
+// over 11 decades) took 15 to 17, and r columns instead of n.  A row of A is a
+// column of A^T, so the pivot is the longest remaining row, and no row is
+// moved: used rows keep their Householder vector.  64 groups of 16 lanes, a
+// row per group; one barrier per step (the norms of the rows' remainders,
+// recomputed in the update, pick the next pivot in every wave).  At 40 x 40 it
+// costs 76 us, and Jacobi and replay fall from 586 + 219 to 189 + 18 us.
+constexpr int kQrpThreads = 1024;
+
+__global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int m, int n,
+                                                          double *Wg, double *Qg) {
+  extern __shared__ double S[];  // m rows of n, padded to ld
+  __shared__ double s_nrm[2][kMaxDim];  // squared norm of the rest, -1: used
+  __shared__ double s_tau[kMaxDim], s_head[kMaxDim], s_alpha[kMaxDim];
+  __shared__ int s_piv[kMaxDim], s_pos[kMaxDim];
+  constexpr int NG = kQrpThreads / 16;
+  const int ld = n | 1;
+  const int r = min(m, n);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int grp = tid >> 4, gl = tid & 15;
+  const double *A = Ag + (int64_t)blockIdx.x * m * n;
+  for (int e = tid; e < m * n; e += kQrpThreads) {
+    const int j = e / n;
+    S[j * ld + (e - j * n)] = A[e];
+  }
+  if (tid < m) s_pos[tid] = r;
+  __syncthreads();
+  for (int j = grp; j < m; j += NG) {
+    double acc = 0.0;
+    for (int i = gl; i < n; i += 16) acc = fma(S[j * ld + i], S[j * ld + i], acc);
+    acc = sum16(acc);
+    if (gl == 0) s_nrm[0][j] = acc;
+  }
+  __syncthreads();
+  for (int k = 0; k < r; ++k) {
+    const double *cur = s_nrm[k & 1];
+    double *next = s_nrm[(k + 1) & 1];
+    // the longest remaining row (the smallest index on a tie)
+    double best = lane < m ? cur[lane] : -2.0;
+    int bj = lane;
+    if (lane + 64 < m && cur[lane + 64] > best) {
+      best = cur[lane + 64];
+      bj = lane + 64;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      const double ov = __shfl_xor(best, o, 64);
+      const int oj = __shfl_xor(bj, o, 64);
+      if (ov > best || (ov == best && oj < bj)) {
+        best = ov;
+        bj = oj;
+      }
+    }
+    bj = __builtin_amdgcn_readfirstlane(bj);
+    // Householder vector of its elements k..n-1 (in place; the head apart)
+    const double *v = S + bj * ld;
+    const double bk = v[k];
+    double al = 0.0, tau = 0.0, head = 0.0;
+    if (best > 0.0) {
+      const double nb = sqrt(best);
+      al = bk > 0.0 ? -nb : nb;
+      head = bk - al;
+      tau = 1.0 / (best + fabs(bk) * nb);
+    }
+    if (tid == 0) {
+      s_tau[k] = tau;
+      s_head[k] = head;
+      s_alpha[k] = al;
+      s_piv[k] = bj;
+      s_pos[bj] = k;
+    }
+    const int i0 = (k & ~15) + gl;
+    for (int j = grp; j < m; j += NG) {
+      const bool live = j != bj && cur[j] >= 0.0;
+      if (live) {
+        double *b = S + j * ld;
+        double dot = 0.0;
+        for (int i = i0; i < n; i += 16) {
+          const double vi = i == k ? head : v[i];
+          if (i >= k) dot = fma(vi, b[i], dot);
+        }
+        const double f = tau * sum16(dot);
+        double rest = 0.0;
+        for (int i = i0; i < n; i += 16) {
+          const double vi = i == k ? head : v[i];
+          if (i >= k) {
+            const double x = fma(-f, vi, b[i]);
+            b[i] = x;
+            if (i > k) rest = fma(x, x, rest);
+          }
+        }
+        rest = sum16(rest);
+        if (gl == 0) next[j] = rest;
+      } else if (gl == 0) {
+        next[j] = -1.0;
+      }
+    }
+    __syncthreads();
+  }
+  // W, column-major: row j holds R's entries up to its pivot step
+  double *W = Wg + (int64_t)blockIdx.x * m * r;
+  for (int e = tid; e < m * r; e += kQrpThreads) {
+    const int c = e / m, j = e - c * m;
+    const int pos = s_pos[j];
+    W[e] = c < pos ? S[j * ld + c] : (c == pos ? s_alpha[c] : 0.0);
+  }
+  if (!Qg) return;
+  // Q = H_0 ... H_{r-1} (unit columns): column c on one group, in registers
+  double *Q = Qg + (int64_t)blockIdx.x * n * r;
+  for (int c = grp; c < r; c += NG) {
+    double q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) q[u] = gl + 16 * u == c ? 1.0 : 0.0;
+    for (int k = c; k >= 0; --k) {
+      const double *v = S + s_piv[k] * ld;
+      const double head = s_head[k];
+      double vv[8], dot = 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = gl + 16 * u;
+        vv[u] = i < k || i >= n ? 0.0 : (i == k ? head : v[i]);
+        dot = fma(vv[u], q[u], dot);
+      }
+      const double f = s_tau[k] * sum16(dot);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = fma(-f, vv[u], q[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (gl + 16 * u < n) Q[(int64_t)(gl + 16 * u) * r + c] = q[u];
+  }
+}
+
 // Round-robin (circle method) pairing for pe (even) players, round s:
 // pair 0 = (s, pe-1); pair k>0 = ((s+k) mod (pe-1), (s-k) mod (pe-1)).
 __device__ __forceinline__ void rr_pair(int s, int k, int pe, int &i, int &j) {
@@ -665,6 +802,25 @@ __device__ __forceinline__ void rr_pair(int s, int k, int pe, int &i, int &j) {
   }
 }
 
+// The rotation that makes columns of squared norms a, bb and inner product g
+// orthogonal (x' = c x - s y, y' = s x + c y): with d = bb - a,
+//   cos 2t = |d| / sqrt(d^2 + 4 g^2), c^2 = (1 + cos 2t) / 2,
+//   s = sign(d) g / (c sqrt(d^2 + 4 g^2)).
+// Two reciprocal square roots instead of two square roots and two divisions
+// (the angle is computed by all 16 lanes of a pair, so it weighs as much as
+// the rotation itself); scaled to a + bb ~ 1 so that the squares neither
+// overflow nor vanish.
+__device__ __forceinline__ void jacobi_angle(double a, double bb, double g, double &c,
+                                             double &s) {
+  const int e = -__builtin_amdgcn_frexp_exp(a + bb);
+  const double d = __builtin_amdgcn_ldexp(bb - a, e), gs = __builtin_amdgcn_ldexp(g, e);
+  const double r1 = rsqrt_newton(fma(d, d, 4.0 * gs * gs));
+  const double c2 = fma(0.5 * fabs(d), r1, 0.5);
+  const double r2 = rsqrt_newton(c2);
+  c = c2 * r2;
+  s = (d < 0.0 ? -gs : gs) * r1 * r2;
+}
+
 // FULL: m == kMaxDim (the randomized path's projected problems), so the
 // row guards of the inner loops are compile-time true.
 template <bool FULL>
@@ -679,8 +835,8 @@ __global__ __launch_bounds__(1024) void jacobi_kernel(
   double *Wb = Wg + (int64_t)b * m * p;
   const int pe = p + (p & 1);  // even number of columns (pad one zero col)
   const int tid = threadIdx.x;
-  double fro = 0.0;
   const int nt = blockDim.x;
+  double big = 0.0;
   for (int i0 = 0; i0 < m * pe; i0 += 8 * nt) {  // 8 loads in flight
     double v[8];
 #pragma unroll
@@ -692,8 +848,23 @@ __global__ __launch_bounds__(1024) void jacobi_kernel(
     for (int u = 0; u < 8; ++u) {
       const int i = i0 + u * nt + tid;
       if (i < m * pe) W[i] = v[u];
-      fro += v[u] * v[u];
+      big = fmax(big, fabs(v[u]));
     }
+  }
+  // scaled by a power of two (exact) to a largest entry in [1, 2): the
+  // products of squared norms in the convergence test neither overflow nor
+  // vanish
+  for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+  if ((tid & 63) == 0) s_off[tid >> 6] = big;
+  __syncthreads();
+  for (int w = 0; w < (nt >> 6); ++w) big = fmax(big, s_off[w]);
+  const int ex = big > 0.0 && big <= DBL_MAX ? __builtin_amdgcn_frexp_exp(big) - 1 : 0;
+  __syncthreads();
+  double fro = 0.0;
+  for (int i = tid; i < m * pe; i += nt) {  // the elements this thread stored
+    const double v = __builtin_amdgcn_ldexp(W[i], -ex);
+    W[i] = v;
+    fro += v * v;
   }
   for (int o = 32; o > 0; o >>= 1) fro += __shfl_xor(fro, o, 64);
   if ((tid & 63) == 0) s_off[tid >> 6] = fro;
@@ -748,13 +919,7 @@ __global__ __launch_bounds__(1024) void jacobi_kernel(
         if (g != 0.0 && a > tiny && bb > tiny && g2 > tol2 * (a * bb)) {
           {
             off_local = 1.0;
-            // t = tan(theta) = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)) with
-            // zeta = (bb - a) / (2 g), multiplied through by |2 g|
-            const double dd = bb - a;
-            const double t = (dd < 0.0 ? -2.0 * g : 2.0 * g) /
-                             (fabs(dd) + sqrt(dd * dd + 4.0 * g2));
-            c = 1.0 / sqrt(1.0 + t * t);
-            sn = c * t;
+            jacobi_angle(a, bb, g, c, sn);
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
               const int r = gl + 16 * u;
@@ -788,9 +953,9 @@ __global__ __launch_bounds__(1024) void jacobi_kernel(
     double acc = 0.0;
     const double *wc = W + jc * m;
     for (int r = 0; r < m; ++r) acc += wc[r] * wc[r];
-    sigma[(int64_t)b * p + jc] = sqrt(acc);
+    sigma[(int64_t)b * p + jc] = __builtin_amdgcn_ldexp(sqrt(acc), ex);
   }
-  for (int i = tid; i < m * p; i += blockDim.x) Wb[i] = W[i];
+  for (int i = tid; i < m * p; i += blockDim.x) Wb[i] = __builtin_amdgcn_ldexp(W[i], ex);
   if (tid == 0 && nsteps) nsteps[b] = steps;
 }
 
@@ -860,10 +1025,7 @@ __global__ __launch_bounds__(1024) void jacobi_big_kernel(
         const double g2 = g * g;
         if (g != 0.0 && a > tiny && bb > tiny && g2 > tol2 * (a * bb)) {
           off_local = 1.0;
-          const double dd = bb - a;
-          const double t = (dd < 0.0 ? -2.0 * g : 2.0 * g) / (fabs(dd) + sqrt(dd * dd + 4.0 * g2));
-          c = 1.0 / sqrt(1.0 + t * t);
-          sn = c * t;
+          jacobi_angle(a, bb, g, c, sn);
 #pragma unroll
           for (int u = 0; u < 16; ++u) {
             const int r = gl + 16 * u;
@@ -900,7 +1062,80 @@ __global__ __launch_bounds__(1024) void jacobi_big_kernel(
   if (tid == 0 && nsteps) nsteps[b] = steps;
 }
 
-// J = I * (product of recorded rotations).  Row-parallel: one 64-lane
+// J = J0 * (product of recorded rotations), p <= 128 columns, J0 (rows x p)
+// given or the identity.  The rows of J are independent: one wave carries a row, lane k the two elements of the round's
+// pair k.  From one round-robin round to the next the first elements of the
+// pairs move one lane down and the second ones one lane up (the last lane
+// turns its second into a first, lane 0 its first into lane 1's second and
+// keeps the fixed column), so a round is four FMAs, one coalesced load of its
+// (c, s) a chunk of rounds ahead, and DPP wave shifts: no LDS and no barrier.
+// 128 rows, 762 rounds: 43 us against 209 us with the rows in LDS.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+__global__ __launch_bounds__(64) void jacobi_replay_kernel(const double *rot, const int *nsteps,
+                                                           int p, const double *J0, double *J) {
+  constexpr int CH = 8;  // rounds per chunk of loads
+  constexpr int kShl = 0x130, kShr = 0x138;  // lane k from k + 1, from k - 1
+  const int np = (p + 1) / 2, q = 2 * np - 1;  // pairs; players but the fixed one
+  const int lane = threadIdx.x, row = blockIdx.x;
+  const bool first = lane == 0, last = lane == np - 1;
+  // round 0: pair k = (k, q - k), pair 0 = (0, q)
+  int ia = lane, ib = lane == 0 ? q : q - lane;
+  double xa, xb;
+  if (J0) {
+    const double *j0 = J0 + (int64_t)row * p;
+    xa = lane < np && ia < p ? j0[ia] : 0.0;
+    xb = lane < np && ib < p ? j0[ib] : 0.0;
+  } else {
+    xa = ia == row ? 1.0 : 0.0;
+    xb = ib == row ? 1.0 : 0.0;
+  }
+  const int ns = __builtin_amdgcn_readfirstlane(nsteps[0]);
+  const double2 *cs = reinterpret_cast<const double2 *>(rot) + min(lane, np - 1);
+  double2 nxt[CH];
+  auto fetch = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u) nxt[u] = cs[(int64_t)min(s0 + u, ns - 1) * np];
+  };
+  auto round = [&](const double2 &r) {
+    // the stream's rotations act on (smaller, larger) column index
+    const double sn = ia < ib ? r.y : -r.y;
+    const double a = xa;
+    xa = fma(r.x, a, -(sn * xb));
+    xb = fma(sn, a, r.x * xb);
+    const double up = dpp_move<kShr>(first ? xa : xb), down = dpp_move<kShl>(xa);
+    xa = np == 1 ? xa : last ? xb : down;
+    xb = first ? xb : up;
+    const int iup = __builtin_amdgcn_mov_dpp(first ? ia : ib, kShr, 0xF, 0xF, true);
+    const int idown = __builtin_amdgcn_mov_dpp(ia, kShl, 0xF, 0xF, true);
+    ia = np == 1 ? ia : last ? ib : idown;
+    ib = first ? ib : iup;
+  };
+  if (ns > 0) fetch(0);
+  int s0 = 0;
+  for (; s0 + CH <= ns; s0 += CH) {
+    double2 cur[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) cur[u] = nxt[u];
+    fetch(s0 + CH);
+#pragma unroll
+    for (int u = 0; u < CH; ++u) round(cur[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < CH; ++u)
+    if (s0 + u < ns) round(nxt[u]);
+  if (lane < np) {
+    if (ia < p) J[(int64_t)row * p + ia] = xa;
+    if (ib < p) J[(int64_t)row * p + ib] = xb;
+  }
+}
+
+// The same for 128 < p <= 256.  Row-parallel: one 64-lane
 // workgroup owns ROWS rows of J in LDS and replays the rotation stream.  The
 // stream is read in chunks of kAccChunk rounds: the next chunk is loaded
 // into registers (independent loads, all in flight) while the current one is
@@ -1015,6 +1250,10 @@ void linalg_init_device() {
       reinterpret_cast<const void *>(&jacobi_kernel<false>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   TN_HIP_CHECK(hipFuncSetAttribute(
+      reinterpret_cast<const void *>(&qrp_kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize,
+      (int)((size_t)kMaxDim * (kMaxDim + 1) * sizeof(double))));
+  TN_HIP_CHECK(hipFuncSetAttribute(
       reinterpret_cast<const void *>(&trsm_ut_kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize,
       (int)((size_t)kTrsmRows * (kTrsmRows + 1) * sizeof(double))));
@@ -1105,18 +1344,28 @@ void jacobi_svd(double *W, int m, int p, int batch, double tol,
   TN_HIP_CHECK(hipGetLastError());
 }
 
+void qrp(const double *A, int m, int n, int batch, double *W, double *Q, hipStream_t s) {
+  TN_REQUIRE(m >= 1 && n >= 1 && m <= kMaxDim && n <= kMaxDim, "qrp: dimension out of range");
+  if (batch <= 0) return;
+  const size_t lds = (size_t)m * (n | 1) * sizeof(double);
+  hipLaunchKernelGGL(qrp_kernel, dim3(batch), dim3(kQrpThreads), lds, s, A, m, n, W, Q);
+  TN_HIP_CHECK(hipGetLastError());
+}
+
 void jacobi_accumulate(const double *rot, const int *nsteps, int p, double *J,
-                       hipStream_t s) {
+                       hipStream_t s, const double *J0, int rows) {
   TN_REQUIRE(p >= 1 && p <= kMaxDimBig, "jacobi_accumulate: p out of range");
-  // 2 rows per workgroup: measured 286 us per 128 x 128 replay at D=5,
-  // chi=100 against 318 us with 4 rows and 394 us with 8
-  constexpr int ROWS = 2;
-  if (p <= kMaxDim)
-    hipLaunchKernelGGL((jacobi_accum_kernel<ROWS, kMaxDim>), dim3(ceil_div(p, ROWS)),
-                       dim3(64), 0, s, rot, nsteps, p, J);
-  else
+  TN_REQUIRE(!J0 || (p <= kMaxDim && rows >= 1), "jacobi_accumulate: start matrix");
+  if (p <= kMaxDim) {
+    hipLaunchKernelGGL(jacobi_replay_kernel, dim3(J0 ? rows : p), dim3(64), 0, s, rot, nsteps, p,
+                       J0, J);
+  } else {
+    // 2 rows per workgroup: 286 us per 128 x 128 replay against 318 us with 4
+    // rows and 394 us with 8 (D=5, chi=100)
+    constexpr int ROWS = 2;
     hipLaunchKernelGGL((jacobi_accum_kernel<ROWS, kMaxDimBig>), dim3(ceil_div(p, ROWS)),
                        dim3(64), 0, s, rot, nsteps, p, J);
+  }
   TN_HIP_CHECK(hipGetLastError());
 }
 

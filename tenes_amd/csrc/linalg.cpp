@@ -36,7 +36,7 @@ double jacobi_tol_for(const SvdOptions &opt, int m) {
 
 // Jacobi SVD of the rows x cols matrix held column-major in W (consumed).
 // Returns sorted sigma (device, length cols), perm (device), J (cols x cols,
-// row-major) if want_J.
+// row-major) if want_J, times J0 (any rows x cols) if given.
 struct JacobiOut {
   Tensor sigma_sorted;
   IntBuf *perm = nullptr;
@@ -50,7 +50,7 @@ struct JacobiOut {
 };
 
 void run_jacobi(Context &ctx, Tensor &W, int rows, int cols, bool want_J,
-                const SvdOptions &opt, JacobiOut &out) {
+                const SvdOptions &opt, JacobiOut &out, const Tensor &J0 = Tensor()) {
   hipStream_t s = ctx.stream();
   const int pe = cols + (cols & 1);
   Tensor sigma = empty(ctx, Shape{cols});
@@ -67,8 +67,10 @@ void run_jacobi(Context &ctx, Tensor &W, int rows, int cols, bool want_J,
   kern::sort_desc(sigma.data(), cols, 1, out.sigma_sorted.data(),
                   out.perm->ptr, s);
   if (want_J) {
-    out.J = empty(ctx, Shape{cols, cols});
-    kern::jacobi_accumulate(rot.data(), nsteps, cols, out.J.data(), s);
+    const int64_t jrows = J0.defined() ? J0.shape[0] : cols;
+    out.J = empty(ctx, Shape{jrows, cols});
+    kern::jacobi_accumulate(rot.data(), nsteps, cols, out.J.data(), s,
+                            J0.defined() ? J0.data() : nullptr, (int)jrows);
   }
   out.W = W;
 }
@@ -291,12 +293,23 @@ SvdPending svd_top_begin_impl(Context &ctx, const Tensor *Ap, const LinearOp *op
     X = transpose(R2, Axes{1, 0});  // B = Q^T A = R2^T Rq^T
   }
 
-  const int rows = (int)X.shape[0], cols = (int)X.shape[1];
-  // Column-major copy of X = row-major X^T.
-  Tensor W = transpose(X, Axes{1, 0});
-  JacobiOut jo;
-  run_jacobi(ctx, W, rows, cols, true, opt, jo);
+  const int rows = (int)X.shape[0];
+  int cols = (int)X.shape[1];
+  const int jrows = cols;
   const int k = std::min(k_target, std::min(rows, cols));
+  JacobiOut jo;
+  if (randomized) {
+    // X comes triangular and graded from the range finder: column-major copy
+    // of X = row-major X^T
+    Tensor W = transpose(X, Axes{1, 0});
+    run_jacobi(ctx, W, rows, cols, true, opt, jo);
+  } else {
+    const int r = std::min(rows, cols);
+    Tensor W = empty(ctx, Shape{r, rows}), Q0 = empty(ctx, Shape{cols, r});
+    kern::qrp(X.data(), rows, cols, 1, W.data(), Q0.data(), s);
+    run_jacobi(ctx, W, rows, r, true, opt, jo, Q0);
+    cols = r;
+  }
 
   // Xhat = W(:,perm)/sigma (rows x k), Jp = J(:,perm) (cols x k)
   Tensor What = empty(ctx, Shape{rows, k});
@@ -304,8 +317,8 @@ SvdPending svd_top_begin_impl(Context &ctx, const Tensor *Ap, const LinearOp *op
                     rows, k, What.data(), s);
   // the randomized path keeps all right Ritz vectors (a warm start block)
   const int kj = randomized ? cols : k;
-  Tensor Jp = empty(ctx, Shape{cols, kj});
-  kern::gather_cols(jo.J.data(), cols, 1, jo.perm->ptr, nullptr, cols, kj,
+  Tensor Jp = empty(ctx, Shape{jrows, kj});
+  kern::gather_cols(jo.J.data(), cols, 1, jo.perm->ptr, nullptr, jrows, kj,
                     Jp.data(), s);
   SvdPending pd;
   SvdResult &r = pd.r;
@@ -367,19 +380,23 @@ Tensor svd_values_batched(Context &ctx, const std::vector<Tensor> &mats) {
              "svd_values_batched: matrices larger than 256 x 256");
   const int b = (int)mats.size();
   hipStream_t s = ctx.stream();
-  // Jacobi acts on the columns of the stored column-major matrix.  Use the
-  // shorter side as the column length: for m >= n store X column-major.
-  const bool tr = m < n;  // then orthogonalise the columns of X^T
-  const int rows = tr ? n : m, cols = tr ? m : n;
+  // Jacobi acts on the columns of the stored column-major matrix.  Up to 128
+  // it is preconditioned (kern::qrp, which leaves min(m, n) columns of length
+  // m); above, the shorter side is the column length: for m >= n store X
+  // column-major, else orthogonalise the columns of X^T.
+  const bool small = m <= kJac && n <= kJac;
+  const bool tr = !small && m < n;
+  const int rows = tr ? n : m, cols = small ? std::min(m, n) : tr ? m : n;
   Tensor W = empty(ctx, Shape{b, cols, rows});
+  Tensor in = small ? empty(ctx, Shape{b, m, n}) : W;
   for (int i = 0; i < b; ++i) {
     TN_REQUIRE(mats[i].shape == mats[0].shape,
                "svd_values_batched: shape mismatch in batch");
-    Tensor src = tr ? mats[i] : transpose(mats[i], Axes{1, 0});
-    TN_HIP_CHECK(hipMemcpyAsync(W.data() + (int64_t)i * rows * cols,
-                                src.data(), sizeof(double) * rows * cols,
-                                hipMemcpyDeviceToDevice, s));
+    Tensor src = small || tr ? mats[i] : transpose(mats[i], Axes{1, 0});
+    TN_HIP_CHECK(hipMemcpyAsync(in.data() + (int64_t)i * m * n, src.data(),
+                                sizeof(double) * m * n, hipMemcpyDeviceToDevice, s));
   }
+  if (small) kern::qrp(in.data(), m, n, b, W.data(), nullptr, s);
   Tensor sigma = empty(ctx, Shape{b, cols});
   SvdOptions opt;
   kern::jacobi_svd(W.data(), rows, cols, b, jacobi_tol_for(opt, rows),

@@ -101,18 +101,18 @@ void svd_small(int device, hipStream_t s, const double *A, int m, int n, int k,
   int *perm = reinterpret_cast<int *>(base + kPerm);
   int *nsteps = reinterpret_cast<int *>(base + kSteps);
   double *rot = base + kRot;
-  // W = A^T row-major = A column-major: the Jacobi kernel orthogonalises the
-  // n columns (length m) of A, as svd_top does on this path
-  const int64_t shape[2] = {n, m}, src[2] = {1, n}, dst[2] = {m, 1};
-  kern::strided_copy(A, W, 2, shape, src, dst, (int64_t)m * n, s);
+  // A = W J^T preconditioned, then the Jacobi on the r columns of W and its
+  // rotations replayed on J in place, as svd_top does on this path
+  const int r = std::min(m, n);
+  kern::qrp(A, m, n, 1, W, J, s);
   const double tol = std::sqrt((double)m) * 2.220446049250313e-16;
-  kern::jacobi_svd(W, m, n, 1, tol, kSweeps, sigma, rot, nsteps, s);
-  kern::sort_desc(sigma, n, 1, sorted, perm, s);
-  kern::jacobi_accumulate(rot, nsteps, n, J, s);
+  kern::jacobi_svd(W, m, r, 1, tol, kSweeps, sigma, rot, nsteps, s);
+  kern::sort_desc(sigma, r, 1, sorted, perm, s);
+  kern::jacobi_accumulate(rot, nsteps, r, J, s, J, n);
   const int kk = std::min(k, std::min(m, n));
   // U = W(:, perm) / sigma (m x kk), V = J(:, perm) (n x kk), s = sorted[:kk]
   kern::gather_cols(W, 1, m, perm, sorted, m, kk, U, s);
-  kern::gather_cols(J, n, 1, perm, nullptr, n, kk, V, s);
+  kern::gather_cols(J, r, 1, perm, nullptr, n, kk, V, s);
   TN_HIP_CHECK(hipMemcpyAsync(sv, sorted, (size_t)kk * sizeof(double),
                               hipMemcpyDeviceToDevice, s));
   if (k_out) *k_out = kk;

@@ -303,3 +303,35 @@ def test_tall_svd_block_edges(gpu_ctx, p, deficient):
     assert np.max(np.abs((U * s) @ V.T - A)) < 3e-13 * ref[0]
     r = p - 2 if deficient and p >= 3 else p
     assert np.max(np.abs(U[:, :r].T @ U[:, :r] - np.eye(r))) < 3e-13
+
+
+@pytest.mark.parametrize("m,p", [(1, 1), (1, 5), (5, 1), (3, 2), (8, 8), (16, 16), (17, 16), (16, 17), (32, 33),
+                                 (33, 32), (40, 40), (64, 64), (65, 63), (63, 65), (100, 128), (128, 100),
+                                 (127, 127), (128, 128)])
+@pytest.mark.parametrize("scale", [1.0, 1e-90, 1e90])
+def test_jacobi_svd_slot_edges(gpu_ctx, m, p, scale):
+    """The one-workgroup Jacobi SVD at the edges of its column slots (16, 32,
+    64, 128) and rows per lane, with a graded spectrum, a repeated singular
+    value and (from 8 columns on) a rank-deficient block, also far from
+    unit scale.  Tolerance: orthogonality is iterated to sqrt(m) eps per
+    pair and the factors accumulate about ten sweeps of rotations: 128 eps
+    times ten, 3e-13."""
+    rng = np.random.default_rng(1000 * m + p)
+    k = min(m, p)
+    q1, _ = np.linalg.qr(rng.standard_normal((m, k)))
+    q2, _ = np.linalg.qr(rng.standard_normal((p, k)))
+    s0 = np.logspace(0, -10, k)
+    if k >= 3:
+        s0[1] = s0[0]
+    if k >= 8:
+        s0[-2:] = 0.0
+    A = (q1 * s0) @ q2.T * scale
+    U, s, V = ta.svd_top(gpu_ctx.tensor(A), k)
+    U, V = U.numpy(), V.numpy()
+    ref = np.linalg.svd(A, compute_uv=False)[:k]
+    assert s.shape == (k,)
+    assert np.max(np.abs(s - ref)) < 3e-13 * ref[0]
+    assert np.max(np.abs((U * s) @ V.T - A)) < 3e-13 * ref[0]
+    assert np.max(np.abs(V.T @ V - np.eye(k))) < 3e-13
+    r = k - 2 if k >= 8 else k
+    assert np.max(np.abs(U[:, :r].T @ U[:, :r] - np.eye(r))) < 3e-13
