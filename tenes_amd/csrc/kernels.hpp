@@ -136,6 +136,11 @@ void splitk_reduce(const double *P, int splits, int M, int N, double alpha,
                    double beta, double *C, const int *c_m, const int *c_n,
                    hipStream_t s);
 
+// Start and end clock of one wave that waits for `ticks` of the device's
+// 100 MHz clock, as two int64 in out (scratch of 16 bytes).
+constexpr int kProbeTicks = 10000;  // 100 us, above the time to launch 8 of them
+void lane_probe(double *out, int ticks, hipStream_t s);
+
 // ---------------------------------------------------------------------------
 // Dense linear algebra building blocks (FP64)
 // ---------------------------------------------------------------------------

@@ -170,6 +170,18 @@ __global__ void gather_cols_kernel(const double *src, int64_t rs, int64_t cs,
   }
 }
 
+__global__ void lane_probe_kernel(long long *out, int ticks) {
+  if (threadIdx.x != 0) return;
+  const long long t0 = wall_clock64();
+  long long t1 = t0;
+  for (int i = 0; i < (1 << 20) && t1 - t0 < ticks; ++i) {  // ends with either bound
+    __builtin_amdgcn_s_sleep(8);
+    t1 = wall_clock64();
+  }
+  out[0] = t0;
+  out[1] = t1;
+}
+
 inline int grid_for(int64_t n) {
   int64_t g = (n + TPB - 1) / TPB;
   if (g > 8192) g = 8192;
@@ -273,6 +285,12 @@ void gather_cols(const double *src, int64_t rs, int64_t cs, const int *perm,
   if (n <= 0) return;
   hipLaunchKernelGGL(gather_cols_kernel, dim3(grid_for(n)), dim3(TPB), 0, s,
                      src, rs, cs, perm, scale, rows, k, out);
+  TN_HIP_CHECK(hipGetLastError());
+}
+
+void lane_probe(double *out, int ticks, hipStream_t s) {
+  hipLaunchKernelGGL(lane_probe_kernel, dim3(1), dim3(64), 0, s,
+                     reinterpret_cast<long long *>(out), ticks);
   TN_HIP_CHECK(hipGetLastError());
 }
 

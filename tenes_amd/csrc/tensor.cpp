@@ -229,6 +229,8 @@ void Context::fork(int n) {
 }
 
 void Context::add_lanes(int n) {
+  const bool first = lanes_.size() == 1;
+  if (first) n = std::max(n, kLanePool);
   while ((int)lanes_.size() < n + 1) {
     Lane l;
     // default priority: every stream of the library runs at one priority
@@ -236,6 +238,44 @@ void Context::add_lanes(int n) {
     TN_HIP_CHECK(hipMalloc(&l.scal, 4096 * sizeof(double)));
     lanes_.push_back(l);
   }
+  if (first) spread_lanes();
+}
+
+// The runtime maps streams onto a few hardware queues (four by default) and
+// work of streams that share one runs in order: the first four side streams
+// of a process came out on two queues, so four projector chains ran two by
+// two (environment runs D=2, chi=10 / D=3, chi=27 / D=5, chi=100: 28 / 91 /
+// 252 ms; on four queues 22 / 69 / 201 ms).  Which streams share a queue
+// cannot be asked, so it is measured once per context: a short clock loop on
+// every lane, and lanes whose intervals overlap go first.  Only the order of
+// the lanes depends on it.
+void Context::spread_lanes() {
+  const int n = (int)lanes_.size() - 1;
+  kern::lane_probe(lanes_[0].scal, 0, lanes_[0].s);  // load the kernel
+  TN_HIP_CHECK(hipStreamSynchronize(lanes_[0].s));
+  for (int i = 1; i <= n; ++i) kern::lane_probe(lanes_[i].scal, kern::kProbeTicks, lanes_[i].s);
+  std::vector<std::array<int64_t, 2>> t(n + 1);
+  for (int i = 1; i <= n; ++i) {
+    TN_HIP_CHECK(hipMemcpyAsync(t[i].data(), lanes_[i].scal, sizeof(t[i]), hipMemcpyDeviceToHost,
+                                lanes_[i].s));
+    TN_HIP_CHECK(hipStreamSynchronize(lanes_[i].s));
+  }
+  auto overlap = [&](int a, int b) { return t[a][0] < t[b][1] && t[b][0] < t[a][1]; };
+  std::vector<int> rest(n), order;
+  std::iota(rest.begin(), rest.end(), 1);
+  while (!rest.empty()) {  // rounds of mutually overlapping lanes
+    std::vector<int> round, left;
+    for (int i : rest) {
+      bool ok = true;
+      for (int j : round) ok = ok && overlap(i, j);
+      (ok ? round : left).push_back(i);
+    }
+    order.insert(order.end(), round.begin(), round.end());
+    rest = left;
+  }
+  std::vector<Lane> sorted(1, lanes_[0]);
+  for (int i : order) sorted.push_back(lanes_[i]);
+  lanes_ = sorted;
 }
 
 void Context::use_lane(int i) {
