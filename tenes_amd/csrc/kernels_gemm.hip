@@ -451,17 +451,55 @@ __global__ void zero_ints_kernel(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
-__global__ void splitk_reduce_kernel(const double *P, int splits, int M, int N,
-                                     double alpha, double beta, double *C,
-                                     const int *c_m, const int *c_n) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// C = alpha sum_z P[z] + beta C.  64 consecutive outputs per block, the
+// splits dealt to its WZ waves and the waves' sums added in wave order (the
+// same sum from launch to launch).  Bound by the latency of each lane's chain
+// of partial loads: with one lane per output, 39 splits of 128 x 128 (5 MB)
+// took 7.3 us, with 16 waves 4.6 us.
+template <int WZ>
+__global__ __launch_bounds__(64 * WZ) void splitk_reduce_kernel(
+    const double *P, int splits, int M, int N, double alpha, double beta, double *C,
+    const int *c_m, const int *c_n) {
+  __shared__ double part[WZ][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t idx = (int64_t)blockIdx.x * 64 + lane;
   const int64_t MN = (int64_t)M * N;
-  if (idx >= MN) return;
   double acc = 0.0;
-  for (int z = 0; z < splits; ++z) acc += P[z * MN + idx];
+  if (idx < MN) {
+#pragma unroll 4
+    for (int z = w; z < splits; z += WZ) acc += P[z * MN + idx];
+  }
+  if (WZ > 1) {
+    part[w][lane] = acc;
+    __syncthreads();
+    if (w != 0) return;
+    acc = part[0][lane];
+#pragma unroll
+    for (int i = 1; i < WZ; ++i) acc += part[i][lane];
+  }
+  if (idx >= MN) return;
   const int m = (int)(idx / N), n = (int)(idx % N);
   double *dst = C + c_m[m] + c_n[n];
   *dst = (beta == 0.0) ? alpha * acc : alpha * acc + beta * (*dst);
+}
+
+// Waves per block: up to four partials per lane are one memory round trip, and
+// a large output has lanes enough on its own.
+void launch_reduce(const double *P, int splits, int M, int N, double alpha, double beta,
+                   double *C, const int *c_m, const int *c_n, hipStream_t s) {
+  const int64_t MN = (int64_t)M * N;
+  const dim3 grid((unsigned)ceil_div(MN, (int64_t)64));
+  const int wz = splits <= 4 ? 1 : splits <= 16 || MN > (1 << 19) ? 4 : 16;
+  if (wz == 1)
+    hipLaunchKernelGGL(splitk_reduce_kernel<1>, grid, dim3(64), 0, s, P, splits, M, N, alpha,
+                       beta, C, c_m, c_n);
+  else if (wz == 4)
+    hipLaunchKernelGGL(splitk_reduce_kernel<4>, grid, dim3(256), 0, s, P, splits, M, N, alpha,
+                       beta, C, c_m, c_n);
+  else
+    hipLaunchKernelGGL(splitk_reduce_kernel<16>, grid, dim3(1024), 0, s, P, splits, M, N,
+                       alpha, beta, C, c_m, c_n);
+  TN_HIP_CHECK(hipGetLastError());
 }
 
 struct Plan {
@@ -524,7 +562,13 @@ Plan choose(int M, int N, int K) {
   // split, fewest splits on a tie.  2500 x 128 x 2500 (80 tiles): 16 splits,
   // 51.5 us against 64.5 us at the 4 that merely reach 256 workgroups.
   p.splits = 1;
-  if (tiles < 128 && K >= 4 * BK * 2) {
+  if (tiles < 8 && K >= 64 * 8 * BK) {
+    // a few tiles and a very long K (density matrices and their gradients,
+    // 32 x 16 x 131072): the operands stream from HBM once, so as many
+    // workgroups as 1024 over the tiles, at least eight K tiles each; 64
+    // splits left three quarters of the CUs idle (165 us, 40 us now)
+    p.splits = std::min(K / (8 * BK), 1024 / (int)tiles);
+  } else if (tiles < 128 && K >= 4 * BK * 2) {
     const int maxs = std::max(1, K / (4 * BK));
     double best = 1e30;
     for (int sp = 1; sp <= std::min(maxs, 64); ++sp) {
@@ -694,24 +738,16 @@ const char *gemm_f64(const GemmArgs &g, void *workspace, size_t ws_bytes,
              : ((p.BM == 128) ? launch_cfg<double, 128, 128>(ka, grid, s)
                               : launch_cfg<double, 64, 64>(ka, grid, s));
   TN_HIP_CHECK(hipGetLastError());
-  if (ka.partial) {
-    const int64_t MN = (int64_t)g.M * g.N;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(ceil_div(MN, 256)),
-                       dim3(256), 0, s, ka.partial, splits, g.M, g.N, g.alpha,
-                       g.beta, g.C, g.c_m, g.c_n);
-    TN_HIP_CHECK(hipGetLastError());
-  }
+  if (ka.partial)
+    launch_reduce(ka.partial, splits, g.M, g.N, g.alpha, g.beta, g.C, g.c_m, g.c_n, s);
   return name;
 }
 
 void splitk_reduce(const double *P, int splits, int M, int N, double alpha,
                    double beta, double *C, const int *c_m, const int *c_n,
                    hipStream_t s) {
-  const int64_t MN = (int64_t)M * N;
-  if (MN == 0) return;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(ceil_div(MN, 256)), dim3(256),
-                     0, s, P, splits, M, N, alpha, beta, C, c_m, c_n);
-  TN_HIP_CHECK(hipGetLastError());
+  if ((int64_t)M * N == 0) return;
+  launch_reduce(P, splits, M, N, alpha, beta, C, c_m, c_n, s);
 }
 
 }  // namespace kern
