@@ -57,8 +57,8 @@ struct GemmPlan {
 bool gemm_stream_k(int M, int N, int K);
 std::vector<GemmPlan> gemm_candidates(int M, int N, int K);
 // Scratch needed for split-K on the given shape (bytes, 0 if none).
-size_t gemm_workspace_bytes(int M, int N, int K,
-                            const GemmPlan *plan = nullptr);
+size_t gemm_workspace_bytes(int M, int N, int K, const GemmPlan *plan = nullptr,
+                            bool f64 = true);
 // Returns the name of the kernel instantiation launched (static string).
 // g.fp32 / g.bf16x3 select the FP32 or the split bf16 MFMA.
 const char *gemm_f64(const GemmArgs &g, void *workspace, size_t ws_bytes,

@@ -537,7 +537,7 @@ bool sk_layout(int M, int N, int K, SkLayout &L) {
   return true;
 }
 
-Plan choose(int M, int N, int K) {
+Plan choose(int M, int N, int K, bool f64) {
   Plan p;
   if (K <= 0) {
     p.BM = p.BN = 64;
@@ -553,6 +553,23 @@ Plan choose(int M, int N, int K) {
   // prologue and epilogue: 2500 x 2500 x 100 in 47 us against 53 us.
   const int64_t tiles128 = (int64_t)ceil_div(M, 128) * ceil_div(N, 128);
   p.BM = p.BN = (M >= 128 && N >= 128 && tiles128 >= 200 && K > 8 * BK) ? 128 : 64;
+  // 32 x 32 tiles (FP64) where the call is a few short workgroups: a K tile
+  // takes 0.34 us in such a workgroup and 0.92 us in a 64 x 64 one (four times
+  // the MFMAs per wave), so up to K = 400 the product needs no split, which
+  // saves the reduction and its launch, and outputs of at most 32 rows or
+  // columns waste less of the tile.  Back to back, with the host's 8.4 us per
+  // call as the floor: 2500 x 128 x 128 13.2 to 8.1 us, 333 x 128 x 333 12.0
+  // to 9.7, 1024 x 1024 x 64 10.4 to 8.4.  Above 2048 tiles the 64 x 64 grid
+  // fills the chip and moves less through L2.
+  const int64_t tiles32 = (int64_t)ceil_div(M, 32) * ceil_div(N, 32);
+  const bool thin = M <= 32 || N <= 32;
+  if (f64 && K <= 400 && (thin || tiles32 <= 2048)) {
+    p.BM = p.BN = 32;
+    p.splits = 1;
+    p.kps = ceil_div(K, BK) * BK;
+    return p;
+  }
+  if (f64 && M <= 32 && N <= 32 && K >= 64 * 8 * BK) p.BM = p.BN = 32;
   const int64_t tiles = (int64_t)ceil_div(M, p.BM) * ceil_div(N, p.BN);
   // Split K when the tile grid cannot fill the 256 CUs and K is long: the
   // split count s that minimises the rounds of 256 workgroups per unit of
@@ -629,10 +646,10 @@ const char *launch_cfg(const KArgs &ka, dim3 grid, hipStream_t s) {
 
 // The heuristic plan, or the given launch shape with its K range rounded
 // to whole tiles (at most one split per K tile).
-Plan plan_for(int M, int N, int K, const GemmPlan *gp) {
-  if (gp == nullptr || gp->bm == 0 || K <= 0) return choose(M, N, K);
+Plan plan_for(int M, int N, int K, const GemmPlan *gp, bool f64 = true) {
+  if (gp == nullptr || gp->bm == 0 || K <= 0) return choose(M, N, K, f64);
   Plan p;
-  p.BM = p.BN = gp->bm == 128 ? 128 : 64;
+  p.BM = p.BN = gp->bm == 128 ? 128 : gp->bm == 32 && f64 ? 32 : 64;
   SkLayout L;
   if (p.BM == 128 && gp->splits == 0 && sk_layout(M, N, K, L)) {
     p.splits = 1;
@@ -656,7 +673,7 @@ bool gemm_stream_k(int M, int N, int K) {
 
 std::vector<GemmPlan> gemm_candidates(int M, int N, int K) {
   std::vector<GemmPlan> out;
-  const Plan h = choose(M, N, K);
+  const Plan h = choose(M, N, K, true);
   auto add = [&](int bm, int splits) {
     if (bm == 128 && (M < 128 || N < 128)) return;
     GemmPlan g{bm, splits};
@@ -679,8 +696,8 @@ std::vector<GemmPlan> gemm_candidates(int M, int N, int K) {
   return out;
 }
 
-size_t gemm_workspace_bytes(int M, int N, int K, const GemmPlan *plan) {
-  Plan p = plan_for(M, N, K, plan);
+size_t gemm_workspace_bytes(int M, int N, int K, const GemmPlan *plan, bool f64) {
+  Plan p = plan_for(M, N, K, plan, f64);
   SkLayout L;
   if (p.sk && sk_layout(M, N, K, L)) return L.bytes;
   if (p.splits <= 1) return 0;
@@ -692,7 +709,7 @@ const char *gemm_f64(const GemmArgs &g, void *workspace, size_t ws_bytes,
   TN_REQUIRE(g.M >= 0 && g.N >= 0 && g.K >= 0, "gemm: negative size");
   if (g.M == 0 || g.N == 0) return "gemm_f64_empty";
   // K == 0 gives C = beta*C through a launch with an empty K range.
-  Plan p = plan_for(g.M, g.N, g.K, plan);
+  Plan p = plan_for(g.M, g.N, g.K, plan, !g.fp32 && !g.bf16x3);
   if (g.bf16x3)
     return gemm_bf16x3(g, p.BM, p.splits, p.kps, workspace, ws_bytes, s);
   KArgs ka;
@@ -735,8 +752,9 @@ const char *gemm_f64(const GemmArgs &g, void *workspace, size_t ws_bytes,
   const char *name =
       g.fp32 ? ((p.BM == 128) ? launch_cfg<float, 128, 128>(ka, grid, s)
                               : launch_cfg<float, 64, 64>(ka, grid, s))
-             : ((p.BM == 128) ? launch_cfg<double, 128, 128>(ka, grid, s)
-                              : launch_cfg<double, 64, 64>(ka, grid, s));
+      : p.BM == 128 ? launch_cfg<double, 128, 128>(ka, grid, s)
+      : p.BM == 32  ? launch_cfg<double, 32, 32>(ka, grid, s)
+                    : launch_cfg<double, 64, 64>(ka, grid, s);
   TN_HIP_CHECK(hipGetLastError());
   if (ka.partial)
     launch_reduce(ka.partial, splits, g.M, g.N, g.alpha, g.beta, g.C, g.c_m, g.c_n, s);

@@ -335,3 +335,32 @@ def test_jacobi_svd_slot_edges(gpu_ctx, m, p, scale):
     assert np.max(np.abs(V.T @ V - np.eye(k))) < 3e-13
     r = k - 2 if k >= 8 else k
     assert np.max(np.abs(U[:, :r].T @ U[:, :r] - np.eye(r))) < 3e-13
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 400), (31, 33, 15), (32, 32, 16), (33, 31, 17), (32, 700, 400),
+                                   (700, 32, 401), (33, 33, 400), (1024, 2048, 31), (1025, 2047, 33),
+                                   (2500, 128, 128), (128, 128, 400), (32, 32, 8191), (32, 32, 8192),
+                                   (9, 18, 18225), (33, 32, 8200), (64, 64, 131072), (200, 130, 9000)])
+@pytest.mark.parametrize("ta_, tb_", [(False, False), (True, False), (False, True), (True, True)])
+def test_matmul_dispatch_edges(gpu_ctx, M, N, K, ta_, tb_):
+    """Both sides of the lines between 32, 64 and 128 tiles, the unsplit, the
+    split and the many-split launch, for the four operand orders, with the
+    mixed-precision modes' own tile choice beside (FP32: its summation bound).
+    FP64 tolerance: 1e-12 of max|C|, as the other products."""
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    A = rng.standard_normal((K, M) if ta_ else (M, K))
+    B = rng.standard_normal((N, K) if tb_ else (K, N))
+    ref = (A.T if ta_ else A) @ (B.T if tb_ else B)
+    a, b = gpu_ctx.tensor(A), gpu_ctx.tensor(B)
+    axes = ([0 if ta_ else 1], [1 if tb_ else 0])
+    C = ta.tensordot(a, b, *axes).numpy()
+    assert _rel(C, ref) < RTOL
+    C2 = ta.tensordot(a, b, *axes, [1, 0]).numpy()
+    assert np.array_equal(C2, C.T)
+    gpu_ctx.set_contraction_mode(1)
+    try:
+        F = ta.tensordot(a, b, *axes).numpy()
+    finally:
+        gpu_ctx.set_contraction_mode(0)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(A.T if ta_ else A) @ np.abs(B.T if tb_ else B))
+    assert np.all(np.abs(F - ref) <= bound + 1e-12)
