@@ -604,14 +604,21 @@ static int affine_stride(const std::vector<int> &tab) {
 const ContractPlan &Context::plan(const Shape &sa, const Shape &sb,
                                   const Axes &axa, const Axes &axb,
                                   const Axes &perm) {
-  std::ostringstream key;
-  key << shape_str(sa) << shape_str(sb) << "|";
-  for (auto a : axa) key << a << ",";
-  key << "|";
-  for (auto a : axb) key << a << ",";
-  key << "|";
-  for (auto a : perm) key << a << ",";
-  auto it = plans_.find(key.str());
+  // looked up for every contraction: the numbers' bytes as the key (an
+  // ostringstream of their digits took longer than the launch)
+  std::string &key = plan_key_;
+  key.clear();
+  auto put = [&key](int64_t v) { key.append(reinterpret_cast<const char *>(&v), sizeof(v)); };
+  put((int64_t)sa.size());
+  for (auto d : sa) put(d);
+  put((int64_t)sb.size());
+  for (auto d : sb) put(d);
+  put((int64_t)axa.size());
+  for (auto x : axa) put(x);
+  put((int64_t)axb.size());
+  for (auto x : axb) put(x);
+  for (auto x : perm) put(x);
+  auto it = plans_.find(key);
   if (it != plans_.end()) return it->second;
   TN_REQUIRE(!capturing_, "tensordot: new contraction plan inside a stream capture");
 
@@ -741,7 +748,7 @@ const ContractPlan &Context::plan(const Shape &sa, const Shape &sb,
   const bool bn1 = p.N > 1 && t_bn[1] - t_bn[0] == 1;
   const bool bk1 = p.K > 1 && t_bk[1] - t_bk[0] == 1;
   p.b_nfast = bn1 && !(bk1 && p.K >= 16 && p.N < 16);
-  return plans_.emplace(key.str(), p).first->second;
+  return plans_.emplace(key, p).first->second;
 }
 
 // ---------------------------------------------------------------------------
@@ -844,12 +851,9 @@ Tensor transpose(const Tensor &t, const Axes &axes) {
   return out;
 }
 
-void tensordot_into(const Tensor &A, const Tensor &B, const Axes &axA,
-                    const Axes &axB, const Axes &perm, Tensor &C, double alpha,
-                    double beta) {
-  Context &ctx = *A.ctx();
-  const ContractPlan &p = ctx.plan(A.shape, B.shape, axA, axB, perm);
-  TN_REQUIRE(C.shape == p.out_shape, "tensordot_into: output shape mismatch");
+// C = alpha A B + beta C by the plan of A's and B's shapes and legs.
+static void contract_into(Context &ctx, const ContractPlan &p, const Tensor &A, const Tensor &B,
+                          Tensor &C, double alpha, double beta) {
   kern::GemmArgs g;
   g.A = A.data();
   g.B = B.data();
@@ -924,13 +928,22 @@ void tensordot_into(const Tensor &A, const Tensor &B, const Axes &axA,
   ctx.gemm_calls++;
 }
 
+void tensordot_into(const Tensor &A, const Tensor &B, const Axes &axA,
+                    const Axes &axB, const Axes &perm, Tensor &C, double alpha,
+                    double beta) {
+  Context &ctx = *A.ctx();
+  const ContractPlan &p = ctx.plan(A.shape, B.shape, axA, axB, perm);
+  TN_REQUIRE(C.shape == p.out_shape, "tensordot_into: output shape mismatch");
+  contract_into(ctx, p, A, B, C, alpha, beta);
+}
+
 Tensor tensordot_t(const Tensor &A, const Tensor &B, const Axes &axA,
                    const Axes &axB, const Axes &perm) {
   TN_REQUIRE(A.defined() && B.defined(), "tensordot: undefined operand");
   Context &ctx = *A.ctx();
   const ContractPlan &p = ctx.plan(A.shape, B.shape, axA, axB, perm);
   Tensor C = make(ctx, p.out_shape);
-  tensordot_into(A, B, axA, axB, perm, C, 1.0, 0.0);
+  contract_into(ctx, p, A, B, C, 1.0, 0.0);
   return C;
 }
 

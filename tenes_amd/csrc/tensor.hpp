@@ -21,6 +21,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "common.hpp"
@@ -333,7 +334,8 @@ class Context {
   hipEvent_t fork_event_ = nullptr;
   double *pinned_ = nullptr;
   double *pinned_dev_ = nullptr;
-  std::map<std::string, ContractPlan> plans_;
+  std::unordered_map<std::string, ContractPlan> plans_;
+  std::string plan_key_;  // of the latest lookup
   uint64_t rng_counter_ = 0;
   int mode_ = 0;
   bool fused_site_ = true;
