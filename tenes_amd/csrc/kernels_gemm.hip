@@ -127,10 +127,12 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
   // when A's m stride is 1) e = ml + BM kl, else (lanes walk k) e = kl + BK ml.
   // Same for B with n.  (ml, kl) and the outer offsets are fixed for the
   // whole K loop and kept in registers.
-  int a_ml[A_PER], a_kl[A_PER], a_moff[A_PER];
-  bool a_mok[A_PER];
-  int b_nl[B_PER], b_kl[B_PER], b_noff[B_PER];
-  bool b_nok[B_PER];
+  // Rows and columns past the edge read row (column) 0: they feed only
+  // outputs that are not stored.  The offset includes the element's k inside
+  // the tile when k is affine, so a load of a full tile is one uniform base
+  // (which moves with the tile) plus a fixed per-thread offset.
+  int a_ml[A_PER], a_kl[A_PER], a_off[A_PER];
+  int b_nl[B_PER], b_kl[B_PER], b_off[B_PER];
   auto setup = [&]() {
 #pragma unroll
     for (int p = 0; p < A_PER; ++p) {
@@ -138,8 +140,8 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
       a_ml[p] = A_MFAST ? e % BM : e / BK;
       a_kl[p] = A_MFAST ? e / BM : e % BK;
       const int m = m0 + a_ml[p];
-      a_mok[p] = m < M;
-      a_moff[p] = a_mok[p] ? (g.a_m_stride ? m * g.a_m_stride : g.a_m[m]) : 0;
+      a_off[p] = (m < M ? (g.a_m_stride ? m * g.a_m_stride : g.a_m[m]) : 0) +
+                 (KA ? a_kl[p] * g.a_k_stride : 0);
     }
 #pragma unroll
     for (int p = 0; p < B_PER; ++p) {
@@ -147,8 +149,8 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
       b_nl[p] = B_NFAST ? e % BN : e / BK;
       b_kl[p] = B_NFAST ? e / BN : e % BK;
       const int n = n0 + b_nl[p];
-      b_nok[p] = n < N;
-      b_noff[p] = b_nok[p] ? (g.b_n_stride ? n * g.b_n_stride : g.b_n[n]) : 0;
+      b_off[p] = (n < N ? (g.b_n_stride ? n * g.b_n_stride : g.b_n[n]) : 0) +
+                 (KB ? b_kl[p] * g.b_k_stride : 0);
     }
   };
 
@@ -174,33 +176,39 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
     }
   };
 
-  // Branch-free tile loads: out-of-range elements read offset 0 (a valid
-  // address) and are replaced by zero only when the tile is stored to LDS,
-  // so all loads of a tile stay in flight during the MFMA work.  Loads and
-  // stores are issued in four parts (part q: elements p with p % 4 == q) so
-  // that the main loop can spread them between its MFMA steps.
+  // Tile loads and stores in four parts (part q: elements p with p % 4 == q)
+  // so that the main loop can spread them between its MFMA steps.  FULL: the
+  // whole tile lies in the K range: no bounds, no selects.  Else elements
+  // past kend are not read and stay zero.  (With a bound and two selects for
+  // every element of every tile the VALU took as many cycles as the MFMAs:
+  // 2500 x 128 x 2500 57 us, 2500 x 2500 x 100 47, 2500^3 744; now 53, 42 and
+  // 724.)
   double ra[A_PER], rb[B_PER];
-  bool oka[A_PER], okb[B_PER];
-  auto load_part = [&](int k0, int q) {
+  auto load_part = [&](auto full, int k0, int q) {
+    constexpr bool FULL = decltype(full)::value;
+    const double *Ak = KA ? g.A + (int64_t)k0 * g.a_k_stride : g.A;
+    const double *Bk = KB ? g.B + (int64_t)k0 * g.b_k_stride : g.B;
 #pragma unroll
     for (int p = 0; p < A_PER; ++p) {
       if (A_PER >= 4 && p % 4 != q) continue;
       if (A_PER < 4 && q != 0) continue;
-      const int kk = a_k_of(k0, p);
-      oka[p] = a_mok[p] && kk < kend;
-      const int koff = KA ? kk * g.a_k_stride : ka_off[A_MFAST ? p : 0];
-      const int off = a_moff[p] + koff;
-      ra[p] = g.A[oka[p] ? off : 0];
+      const int off = a_off[p] + (KA ? 0 : ka_off[A_MFAST ? p : 0]);
+      if (FULL) {
+        ra[p] = Ak[off];
+      } else {
+        ra[p] = a_k_of(k0, p) < kend ? Ak[off] : 0.0;
+      }
     }
 #pragma unroll
     for (int p = 0; p < B_PER; ++p) {
       if (B_PER >= 4 && p % 4 != q) continue;
       if (B_PER < 4 && q != 0) continue;
-      const int kk = b_k_of(k0, p);
-      okb[p] = b_nok[p] && kk < kend;
-      const int koff = KB ? kk * g.b_k_stride : kb_off[B_NFAST ? p : 0];
-      const int off = b_noff[p] + koff;
-      rb[p] = g.B[okb[p] ? off : 0];
+      const int off = b_off[p] + (KB ? 0 : kb_off[B_NFAST ? p : 0]);
+      if (FULL) {
+        rb[p] = Bk[off];
+      } else {
+        rb[p] = b_k_of(k0, p) < kend ? Bk[off] : 0.0;
+      }
     }
   };
   auto store_part = [&](int buf, int q) {
@@ -208,15 +216,17 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
     for (int p = 0; p < A_PER; ++p) {
       if (A_PER >= 4 && p % 4 != q) continue;
       if (A_PER < 4 && q != 0) continue;
-      As[buf][a_kl[p]][a_ml[p]] = (CT)(oka[p] ? ra[p] : 0.0);
+      As[buf][a_kl[p]][a_ml[p]] = (CT)ra[p];
     }
 #pragma unroll
     for (int p = 0; p < B_PER; ++p) {
       if (B_PER >= 4 && p % 4 != q) continue;
       if (B_PER < 4 && q != 0) continue;
-      Bs[buf][b_kl[p]][b_nl[p]] = (CT)(okb[p] ? rb[p] : 0.0);
+      Bs[buf][b_kl[p]][b_nl[p]] = (CT)rb[p];
     }
   };
+  constexpr std::true_type full{};
+  constexpr std::false_type edge{};
 
   acc_t acc[TM][TN];
   const int li = lane & 15;  // row (A) / column (B) inside a 16x16 block
@@ -240,18 +250,18 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
     if (kbeg < kend) {
       fetch_koff(kbeg);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) load_part(kbeg, q);
+      for (int q = 0; q < 4; ++q) load_part(edge, kbeg, q);
 #pragma unroll
       for (int q = 0; q < 4; ++q) store_part(0, q);
       fetch_koff(kbeg + BK);
     }
     __syncthreads();
     int buf = 0;
-    for (int k0 = kbeg; k0 < kend; k0 += BK) {
-      const bool next = k0 + BK < kend;
+    auto step = [&](auto next_full, int k0) {
+      const bool next = decltype(next_full)::value || k0 + BK < kend;
       if (next) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) load_part(k0 + BK, q);
+        for (int q = 0; q < 4; ++q) load_part(next_full, k0 + BK, q);
         fetch_koff(k0 + 2 * BK);
       }
 #pragma unroll
@@ -272,7 +282,10 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
       }
       __syncthreads();
       buf ^= 1;
-    }
+    };
+    int k0 = kbeg;
+    for (; k0 + 2 * BK <= kend; k0 += BK) step(full, k0);
+    for (; k0 < kend; k0 += BK) step(edge, k0);
   } else {
   // Pipeline: tile t is multiplied from LDS buffer t&1 while tile t+1 (in
   // registers since the previous tile) is stored into the other buffer and
@@ -282,19 +295,25 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
   // no branches: past the end of the K range the loads are masked (zeros
   // stored into the buffer no later tile reads).
   if (kbeg < kend) {
-    fetch_koff(kbeg);
+    auto start = [&](auto two_full) {
+      fetch_koff(kbeg);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) load_part(kbeg, q);
+      for (int q = 0; q < 4; ++q) load_part(two_full, kbeg, q);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) store_part(0, q);
-    fetch_koff(kbeg + BK);
+      for (int q = 0; q < 4; ++q) store_part(0, q);
+      fetch_koff(kbeg + BK);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) load_part(kbeg + BK, q);
-    fetch_koff(kbeg + 2 * BK);
+      for (int q = 0; q < 4; ++q) load_part(two_full, kbeg + BK, q);
+      fetch_koff(kbeg + 2 * BK);
+    };
+    if (kbeg + 2 * BK <= kend)
+      start(full);
+    else
+      start(edge);
   }
   __syncthreads();
   int buf = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
+  auto step = [&](auto ahead_full, int k0) {
 #pragma unroll
     for (int ks = 0; ks < BK / 4; ++ks) {
       CT a[TM], b[TN];
@@ -307,7 +326,7 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = Mfma<CT>::run(a[i], b[j], acc[i][j]);
       store_part(buf ^ 1, ks);
-      load_part(k0 + 2 * BK, ks);
+      load_part(ahead_full, k0 + 2 * BK, ks);
       // keep the parts in program order: the compiler would otherwise hoist
       // all stores (and their waits on the loads) to the top of the tile
       __builtin_amdgcn_sched_barrier(0);
@@ -315,7 +334,10 @@ __global__ __launch_bounds__(256, SK ? 2 : 1) void gemm_kernel(KArgs ka) {
     fetch_koff(k0 + 3 * BK);
     __syncthreads();
     buf ^= 1;
-  }
+  };
+  int k0 = kbeg;
+  for (; k0 + 3 * BK <= kend; k0 += BK) step(full, k0);
+  for (; k0 < kend; k0 += BK) step(edge, k0);
   }
   };
 
