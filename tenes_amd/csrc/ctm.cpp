@@ -170,14 +170,19 @@ tensor fused_site(const tensor &X, const tensor &Tn, int legA, int legB, bool ed
   a.Df = (int)X.shape[1];
   a.D = D;
   a.p = (int)Tn.shape[4];
-  // operand arrays (real tensors: the bra is the ket)
-  const tensor TK = tn::transpose(Tn, Axes{legA, legB, 4, o[0], o[1]});
-  const tensor TB = tn::transpose(Tn, Axes{legA, legB, o[0], o[1], 4});
+  // the site tensor as it is, by strides (real tensors: the bra is the ket)
+  int st[5];
+  st[4] = 1;
+  for (int l = 3; l >= 0; --l) st[l] = st[l + 1] * (int)Tn.shape[l + 1];
+  a.sA = st[legA];
+  a.sB = st[legB];
+  a.s0 = st[o[0]];
+  a.s1 = st[o[1]];
+  a.sp = st[4];
   tensor out = edge ? tn::empty(ctx, Shape{a.Ds, a.Df, D, D, D, D})
                     : tn::empty(ctx, Shape{D, a.Ds, D, D, a.Df, D});
   a.X = X.data();
-  a.TK = TK.data();
-  a.TB = TB.data();
+  a.T = Tn.data();
   a.out = out.data();
   tn::kern::site_apply(a, edge, ctx.stream());
   return out;

@@ -80,8 +80,10 @@ const char *gemm_bf16x3(const GemmArgs &g, int bm, int splits, int k_per_split,
 // ---------------------------------------------------------------------------
 struct SiteArgs {
   const double *X;
-  const double *TK;
-  const double *TB;
+  const double *T;  // the site tensor
+  // its strides: the legs met by (kA, bA) and (kB, bB), the legs kept as
+  // (oA, boA) and (oB, boB), the physical leg
+  int sA, sB, s0, s1, sp;
   double *out;
   int Ds, Df, D, p;
 };
@@ -111,8 +113,8 @@ void strided_copy(const double *src, double *dst, int rank,
 void max_abs(const double *x, int64_t n, double *out, double *partials,
              hipStream_t s);
 int max_abs_partials(int64_t n);
-// x[i] /= *d  (d is a device scalar)
-void scale_by_inv(double *x, int64_t n, const double *d, hipStream_t s);
+// x /= max |x| (partials: max_abs_partials(n) doubles)
+void normalize_max(double *x, int64_t n, double *partials, hipStream_t s);
 void scale(double *x, int64_t n, double a, hipStream_t s);
 // out[0] = sum_i x[i]*y[i]
 void dot(const double *x, const double *y, int64_t n, double *out,

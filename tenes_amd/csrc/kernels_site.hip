@@ -35,6 +35,20 @@ namespace {
 constexpr int kSiteThreads = 256;
 constexpr int kSiteNB = 4;
 
+// Elements of the two operand matrices, read from the site tensor by its
+// strides (the tensor, at most 10 KB, stays in cache; two transposed copies
+// cost two launches of 3 to 4 us before every call of this kernel).
+template <int D, int P>
+__device__ __forceinline__ double tb_elem(const SiteArgs &a, int i, int c) {
+  const int bo = c / P, p = c - bo * P;
+  return a.T[(i / D) * a.sA + (i % D) * a.sB + (bo / D) * a.s0 + (bo % D) * a.s1 + p * a.sp];
+}
+template <int D, int P>
+__device__ __forceinline__ double tk_elem(const SiteArgs &a, int k, int o) {
+  const int ki = k / P, p = k - ki * P;
+  return a.T[(ki / D) * a.sA + (ki % D) * a.sB + (o / D) * a.s0 + (o % D) * a.s1 + p * a.sp];
+}
+
 // Store the NB staged output blocks os[q][(oA,oB)][(boA,boB)] of workgroup
 // (s, f0) in the edge (block-major) or corner layout.
 template <bool EDGE, int D, int NT = kSiteThreads>
@@ -97,11 +111,11 @@ __global__ __launch_bounds__(kSiteThreads) void site_apply_kernel(SiteArgs a) {
   const int cb = t % NCB, gb = t / NCB;
   double tb[BI];
 #pragma unroll
-  for (int i = 0; i < BI; ++i) tb[i] = gb < GB ? a.TB[i * NCB + cb] : 0.0;
+  for (int i = 0; i < BI; ++i) tb[i] = gb < GB ? tb_elem<D, P>(a, i, cb) : 0.0;
   const int co = t % KO, gc = t / KO;
   double tk[KI * P];
 #pragma unroll
-  for (int i = 0; i < KI * P; ++i) tk[i] = gc < GC ? a.TK[i * KO + co] : 0.0;
+  for (int i = 0; i < KI * P; ++i) tk[i] = gc < GC ? tk_elem<D, P>(a, i, co) : 0.0;
   __syncthreads();
 
   for (int q = 0; q < nb; ++q) {
@@ -190,7 +204,7 @@ __global__ __launch_bounds__(kSiteMfmaThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int ks = 0; ks < KS1; ++ks) {
       const int k = 4 * ks + lk;
-      b1[ks] = (k < BI && c < NCB) ? a.TB[k * NCB + c] : 0.0;
+      b1[ks] = (k < BI && c < NCB) ? tb_elem<D, P>(a, k, c) : 0.0;
     }
   }
   double a2[MT2][KS2];
@@ -200,7 +214,7 @@ __global__ __launch_bounds__(kSiteMfmaThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int ks = 0; ks < KS2; ++ks) {
       const int k = 4 * ks + lk;
-      a2[mt][ks] = (k < KI * P && m < KO) ? a.TK[k * KO + m] : 0.0;
+      a2[mt][ks] = (k < KI * P && m < KO) ? tk_elem<D, P>(a, k, m) : 0.0;
     }
   }
   __syncthreads();

@@ -1041,11 +1041,9 @@ double max_abs(const Tensor &t) {
 
 void normalize_max_abs(Tensor &t) {
   Context &ctx = *t.ctx();
-  double *d = ctx.scalars(1);
   const int np = kern::max_abs_partials(t.size());
   double *part = static_cast<double *>(ctx.workspace(np * sizeof(double)));
-  kern::max_abs(t.data(), t.size(), d, part, ctx.stream());
-  kern::scale_by_inv(t.data(), t.size(), d, ctx.stream());
+  kern::normalize_max(t.data(), t.size(), part, ctx.stream());
 }
 
 void multiply_vector_dev(Tensor &t, const double *v_dev, int axis) {

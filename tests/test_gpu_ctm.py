@@ -859,3 +859,22 @@ def test_paired_move_chains_equal_reference_order(gpu_ctx):
     Ea, _ = observables_gpu(a, lat, ham)
     Eb, _ = observables_gpu(b, lat, ham)
     assert abs(Ea - Eb) < 1e-12 * abs(Ea)
+
+
+@pytest.mark.parametrize("chi,D", [(1, 2), (4, 2), (20, 2), (64, 2), (65, 2), (27, 5), (100, 2), (40, 4)])
+def test_next_ctm_normalisation_edges(gpu_ctx, chi, D):
+    """The normalisation of Calc_Next_CTM and Calc_Next_eT on both sides of
+    its one-workgroup limit of 16384 elements (chi^2 D^2: 64, 65 at D = 2; 27
+    at D = 5): the largest element is 1 in absolute value and the
+    tensors equal the oracle's to 1e-11."""
+    rng = np.random.default_rng(chi * 10 + D)
+    eT, Tn, PU, PL = random_env_pieces(rng, chi, D)
+    C1, C4 = rng.standard_normal((chi, chi)), rng.standard_normal((chi, chi))
+    t = gpu_ctx.tensor
+    e = ta.calc_next_et(t(eT), t(Tn), t(PU), t(PL)).numpy()
+    a, b = (x.numpy() for x in ta.calc_next_ctm(t(C1), t(C4), t(eT), t(eT), t(PU), t(PL)))
+    assert rel(e, O.Calc_Next_eT(eT, Tn, PU, PL)) < 1e-11
+    ra, rb = O.Calc_Next_CTM(C1, C4, eT, eT, PU, PL)
+    assert rel(a, ra) < 1e-11 and rel(b, rb) < 1e-11
+    for x in (e, a, b):
+        assert abs(np.max(np.abs(x)) - 1.0) < 1e-15
