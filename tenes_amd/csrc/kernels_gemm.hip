@@ -10,7 +10,8 @@
 // transpose into the epilogue store.  When a table is an arithmetic
 // progression the loader computes the offset directly (affine fast path).
 //
-// Tiling: 256 threads = 4 waves (2 x 2), block tile BM x BN x 16, each wave
+// Tiling: 256 threads = 4 waves (2 x 2), block tile BM x BN x 16 (128, 64 or,
+// in FP64, 32 square), each wave
 // owns (BM/2) x (BN/2) = (BM/32) x (BN/32) MFMA 16x16 accumulator tiles.
 // K tiles are staged through LDS with a register prefetch of the next tile.
 // An FP64 16x16x4 MFMA does 2048 flop; at the 78.6 TFLOP/s FP64 matrix peak

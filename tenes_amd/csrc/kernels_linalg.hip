@@ -13,6 +13,8 @@
 //                       is streamed to HBM so the accumulated right factor can
 //                       be rebuilt row-parallel afterwards (jacobi_accumulate)
 //                       without keeping a second p x p matrix in LDS.
+//  * qrp              : row-pivoted QR, the preconditioner of the exact path's
+//                       Jacobi (m, n <= 128).
 //  * sort_desc        : rank sort of singular values, descending.
 #include <cfloat>
 #include <type_traits>

@@ -2,7 +2,7 @@
 // Jacobi on the whole matrix) without any device allocation, for callers
 // that cannot allocate device memory.  Its scratch -- the column-major work
 // copy, the Jacobi rotation stream, the singular values before and after
-// sorting, the permutation, the round count and the accumulated rotations --
+// sorting, the permutation, the round count and the right factor --
 // lives in one file-scope device array of fixed size.  Every region is
 // written before it is read within a call, so nothing needs clearing between
 // calls; calls that overlap on one device share the array and race.
