@@ -107,7 +107,7 @@ __global__ void refill_columns_kernel(double *X, int64_t n, int p,
 //      waves do the rest of the trailing update on the FP64 MFMA.
 // Alone on the device, average over a projector's calls at 128 x 128: 93 us
 // before (4 waves, pivots through LDS with a division each, substitutions
-// through LDS broadcasts, the inverse after the factor), 39 us now; 8 x 8:
+// through LDS broadcasts, the inverse after the factor), 40 us now; 8 x 8:
 // 14.8 us before, 5.6 us now.
 // ---------------------------------------------------------------------------
 constexpr int kCholThreads = 512;

@@ -251,8 +251,8 @@ void Context::add_lanes(int n) {
 // the lanes depends on it.
 void Context::spread_lanes() {
   const int n = (int)lanes_.size() - 1;
-  kern::lane_probe(lanes_[0].scal, 0, lanes_[0].s);  // load the kernel
-  TN_HIP_CHECK(hipStreamSynchronize(lanes_[0].s));
+  kern::lane_probe(lanes_[1].scal, 0, lanes_[1].s);  // load the kernel
+  TN_HIP_CHECK(hipStreamSynchronize(lanes_[1].s));
   for (int i = 1; i <= n; ++i) kern::lane_probe(lanes_[i].scal, kern::kProbeTicks, lanes_[i].s);
   std::vector<std::array<int64_t, 2>> t(n + 1);
   for (int i = 1; i <= n; ++i) {
