@@ -175,9 +175,7 @@ typedef struct tenes_peps_parameters {
    * finder starts from the right Ritz basis the same projector (environment,
    * move, coordinate, row) produced in its previous sweep, kept across
    * tenes_calc_ctm_environment calls that continue an environment
-   * (initialize = 0), with svd_warm_power_iters iterations; with the cut on
-   * the host from the sweep on whose kept singular values agree with the
-   * previous ones to a tenth (a Gaussian block before); start columns
+   * (initialize = 0), with svd_warm_power_iters iterations; start columns
    * that are exactly zero (rank-deficient earlier sweeps) are replaced by
    * Gaussian ones.  Defaults: 1, 8 (svd_power_iters: 8). */
   int svd_warm_start;

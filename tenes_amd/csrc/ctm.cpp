@@ -257,20 +257,6 @@ int r_contraction_mode(const PEPS_Parameters &pp) {
   return pp.contraction_fp32 == 3 ? 2 : (pp.contraction_fp32 == 2 ? 1 : 0);
 }
 
-// Whether a projector's kept singular values moved by less than a tenth
-// since its previous sweep (values below 1e-10 of the first, near the cut and
-// the rounding level, aside): then its Ritz basis may start the next one.
-void note_spectrum(tn::Context::SvdStart &st, const std::vector<double> &s) {
-  std::vector<double> now(s.size());
-  for (size_t i = 0; i < s.size(); ++i) now[i] = s[0] > 0.0 ? s[i] / s[0] : 0.0;
-  st.settled = !now.empty() && st.spectrum.size() == now.size();
-  for (size_t i = 0; st.settled && i < now.size(); ++i) {
-    const double hi = std::max(now[i], st.spectrum[i]), lo = std::min(now[i], st.spectrum[i]);
-    if (hi > 1e-10 && !(lo > 0.9 * hi)) st.settled = false;
-  }
-  st.spectrum = std::move(now);
-}
-
 // From the SVD of the (rows x cols) matrix `Rm`, build the oblique projector
 // pair: PU = Bblk * (VT_c^dagger s^-1/2), PL = Ablk * (U_c^* s^-1/2), both
 // transposed to (e_in, t, tc, cut) (ctm.cpp:290-301 / 466-475).
@@ -293,14 +279,7 @@ void projectors_begin(tn::Context &ctx, const tensor &Rm, int64_t r0,
   if (warm) {
     wkey = {(*key)[0], (*key)[1], (*key)[2], (*key)[3], nc};
     auto it = ctx.svd_start.find(wkey);
-    // The old basis serves once the environment has settled.  Before that
-    // (a growing or turning chi index) its vectors sit in a few symmetry
-    // sectors or index blocks of the new matrix, and directions missing from
-    // them enter only as rounding noise: corner spectra of the second sweep
-    // (Heisenberg, D=5, chi=100, ten seeds) came out 1e-13 to 3e-5 off, and
-    // 5e-15 from a Gaussian block.  (With the cut on the device the values
-    // are not known here, and captured sweeps need one decision.)
-    if (it != ctx.svd_start.end() && (job.device_cut || it->second.settled)) {
+    if (it != ctx.svd_start.end()) {
       opts.start = &it->second.V;
       opts.start_sigma = &it->second.s;
       opts.start_range = it->second.range;
@@ -311,10 +290,7 @@ void projectors_begin(tn::Context &ctx, const tensor &Rm, int64_t r0,
               : tn::svd_top_begin(ctx, tn::reshape(Rm, Shape{nr, nc}), job.kmax, opts, slot);
   job.warm_store = warm && job.sv.r.Vbasis.defined();
   if (job.warm_store) {
-    tn::Context::SvdStart &st = ctx.svd_start[wkey];
-    st.V = job.sv.r.Vbasis;
-    st.s = job.sv.r.sbasis;
-    st.range = 0.0;
+    ctx.svd_start[wkey] = {job.sv.r.Vbasis, job.sv.r.sbasis, 0.0};
     job.wkey = wkey;
   }
   job.slot = slot;
@@ -374,12 +350,10 @@ void projectors_finish(tn::Context &ctx, ProjectorJob &job,
   tn::SvdResult sv = tn::svd_top_end(job.sv);
   if (job.warm_store && !sv.s_all.empty()) {
     auto it = ctx.svd_start.find(job.wkey);
-    if (it != ctx.svd_start.end()) {
+    if (it != ctx.svd_start.end())
       it->second.range = sv.s_all.back() > 0.0
                              ? sv.s_all.front() / sv.s_all.back()
                              : 0.0;
-      note_spectrum(it->second, sv.s);
-    }
   }
   std::vector<double> s_c;
   const int cut0 = std::min<int>(job.kmax, (int)sv.s.size());

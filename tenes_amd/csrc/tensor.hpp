@@ -247,10 +247,6 @@ class Context {
   struct SvdStart {
     Tensor V, s;
     double range = 0.0;
-    // host cut: the kept singular values over the first, and whether the
-    // two latest sweeps' agree (projectors_finish)
-    std::vector<double> spectrum;
-    bool settled = false;
   };
   std::map<std::array<int64_t, 5>, SvdStart> svd_start;
   void forget_svd_starts(int64_t environment);

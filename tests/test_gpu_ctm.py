@@ -654,6 +654,37 @@ def test_ctm_warm_start_rank_growth(gpu_ctx):
         assert worst < 1e-10, (split, worst)
 
 
+@pytest.mark.parametrize("device_cut", [0, 1])
+def test_warm_block_from_the_second_sweep_on(device_cut):
+    """svd_warm_start: the second sweep's range finder starts from the first
+    sweep's basis, on whichever side the cut is made and however far the
+    environment still moves.  Random D=3, chi=27 tensors (243 x 243
+    projector matrices, chi still growing): the iterations of a warm block are
+    svd_warm_power_iters, so 0 of them change the second sweep's corner
+    spectra and the default does not differ from the first sweep's 8; with
+    svd_warm_start = 0 the parameter is not read.  Bitwise comparisons: each
+    run has its own context, seed and launch sequence."""
+    Tn = random_tensors(3, 2, seed=23)
+
+    def spectra(**kw):
+        ctx = ta.Context(0, seed=9)
+        genv = ta.Environment(ctx, 2, 2)
+        genv.set_site_tensors(Tn)
+        genv.calc_ctm_environment(ta.peps_parameters(CHI=27, CTM_Convergence_Epsilon=0.0,
+                                                     projector_cut_on_device=device_cut, **kw))
+        return [genv.corner_spectrum(k, i) for i in range(4) for k in ("C1", "C2", "C3", "C4")]
+
+    def same(a, b):
+        return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+    first = [spectra(Max_CTM_Iteration=1, svd_warm_power_iters=q) for q in (0, 8)]
+    assert same(*first)
+    second = [spectra(Max_CTM_Iteration=2, svd_warm_power_iters=q) for q in (0, 8)]
+    assert not same(*second)
+    cold = [spectra(Max_CTM_Iteration=2, svd_warm_start=0, svd_warm_power_iters=q) for q in (0, 8)]
+    assert same(*cold)
+
+
 def test_afh_real_correlation_functions_on_gpu(gpu_ctx):
     """Correlation functions <Sz(0) Sz(r)>, <Sz(0) Sx(r)>, r = 1..3 along +x
     and +y from every site, and the four-site SzSzSzSz observables on the 2x2
