@@ -211,7 +211,8 @@ void jacobi_accumulate(const double *rot, const int *nsteps, int p, double *J,
 // r = min(m, n)) with columns of falling length, Q (n x r row-major)
 // orthonormal columns, or nullptr.
 void qrp(const double *A, int m, int n, int batch, double *W, double *Q, hipStream_t s);
-// sorted[b][r] = sigma[b][perm[b][r]], descending (ties keep index order).
+// sorted[b][r] = sigma[b][perm[b][r]], descending (ties keep index order, NaN
+// last: perm is a permutation whatever the values).
 void sort_desc(const double *sigma, int p, int batch, double *sorted,
                int *perm, hipStream_t s);
 // One-time per-device kernel attribute setup (large dynamic LDS).

@@ -15,13 +15,14 @@
 //                       without keeping a second p x p matrix in LDS.
 //  * qrp              : row-pivoted QR, the preconditioner of the exact path's
 //                       Jacobi (m, n <= 128).
-//  * sort_desc        : rank sort of singular values, descending.
+//  * sort_desc        : rank sort of singular values, descending (rank.hpp).
 #include <cfloat>
 #include <type_traits>
 #include <utility>
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "rank.hpp"
 
 namespace tn {
 namespace kern {
@@ -1221,10 +1222,7 @@ __global__ void sort_desc_kernel(const double *sigma, int p, int batch,
   for (int j = threadIdx.x; j < p; j += blockDim.x) {
     const double v = sv[j];
     int rank = 0;
-    for (int k = 0; k < p; ++k) {
-      const double u = sv[k];
-      rank += (u > v) || (u == v && k < j);
-    }
+    for (int k = 0; k < p; ++k) rank += ranks_before(sv[k], k, v, j);
     sorted[(int64_t)b * p + rank] = v;
     perm[(int64_t)b * p + rank] = j;
   }
