@@ -141,7 +141,8 @@ int tenes_tensordot(const tenes_tensor *A, const tenes_tensor *B, int nax,
 int tenes_transpose(const tenes_tensor *T, const int *axes, tenes_tensor **out);
 /* Leading k singular triplets of a 2-D tensor (mptensor svd at
  * src/iTPS/core/ctm.cpp:273).  U: (m, k), V: (n, k), s: k values, descending.
- * *k_out receives the number returned. */
+ * *k_out receives the number returned.  With a NaN or an infinite entry in a
+ * matrix of at most 128 x 128 every singular value is NaN. */
 int tenes_svd_top(const tenes_tensor *A, int k, int power_iters,
                   tenes_tensor **U, tenes_tensor **V, double *s, int *k_out);
 /* tenes_svd_top for a matrix of at most 128 x 128 (its exact one-sided

@@ -672,12 +672,24 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
   const int tid = threadIdx.x, lane = tid & 63;
   const int grp = tid >> 4, gl = tid & 15;
   const double *A = Ag + (int64_t)blockIdx.x * m * n;
+  double *W = Wg + (int64_t)blockIdx.x * m * r;
+  double *Q = Qg ? Qg + (int64_t)blockIdx.x * n * r : nullptr;
+  bool finite = true;
   for (int e = tid; e < m * n; e += kQrpThreads) {
     const int j = e / n;
-    S[j * ld + (e - j * n)] = A[e];
+    const double v = A[e];
+    finite = finite && fabs(v) <= DBL_MAX;
+    S[j * ld + (e - j * n)] = v;
   }
   if (tid < m) s_pos[tid] = r;
-  __syncthreads();
+  // a NaN or infinite entry: every value and vector of this matrix is NaN
+  // (below, a NaN norm would be taken for the norm of a zero row)
+  if (__syncthreads_or(!finite)) {
+    const double nan = __builtin_nan("");
+    for (int e = tid; e < m * r; e += kQrpThreads) W[e] = nan;
+    for (int e = tid; Q && e < n * r; e += kQrpThreads) Q[e] = nan;
+    return;
+  }
   for (int j = grp; j < m; j += NG) {
     double acc = 0.0;
     for (int i = gl; i < n; i += 16) acc = fma(S[j * ld + i], S[j * ld + i], acc);
@@ -750,15 +762,13 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
     __syncthreads();
   }
   // W, column-major: row j holds R's entries up to its pivot step
-  double *W = Wg + (int64_t)blockIdx.x * m * r;
   for (int e = tid; e < m * r; e += kQrpThreads) {
     const int c = e / m, j = e - c * m;
     const int pos = s_pos[j];
     W[e] = c < pos ? S[j * ld + c] : (c == pos ? s_alpha[c] : 0.0);
   }
-  if (!Qg) return;
+  if (!Q) return;
   // Q = H_0 ... H_{r-1} (unit columns): column c on one group, in registers
-  double *Q = Qg + (int64_t)blockIdx.x * n * r;
   for (int c = grp; c < r; c += NG) {
     double q[8];
 #pragma unroll

@@ -337,6 +337,30 @@ def test_jacobi_svd_slot_edges(gpu_ctx, m, p, scale):
     assert np.max(np.abs(U[:, :r].T @ U[:, :r] - np.eye(r))) < 3e-13
 
 
+@pytest.mark.parametrize("m,n,at", [(1, 1, (0, 0)), (1, 9, (0, 8)), (9, 1, (0, 0)), (9, 1, (8, 0)), (5, 7, (0, 0)),
+                                    (3, 40, (2, 39)), (40, 40, (0, 3)), (128, 128, (127, 127)), (128, 70, (64, 0))])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_exact_svd_reports_non_finite_input(gpu_ctx, m, n, at, bad):
+    """One NaN or infinite entry in a matrix of the exact path, in the first
+    row (the first pivot of its QR), in a row that is never a pivot and in a
+    column past min(m, n): every singular value is NaN, in the SVD and in the
+    batched values (a corner's spectrum); the next matrix is not affected."""
+    rng = np.random.default_rng(m + n)
+    A = rng.standard_normal((m, n))
+    k = min(m, n)
+    good = np.linalg.svd(A, compute_uv=False)
+    B = A.copy()
+    B[at] = bad
+    U, s, V = ta.svd_top(gpu_ctx.tensor(B), k)
+    assert s.shape == (k,) and np.all(np.isnan(s))
+    assert np.all(np.isnan(V.numpy()))
+    env = ta.Environment(gpu_ctx, 1, 1)
+    env.set("C1", 0, B)
+    assert np.all(np.isnan(env.corner_spectrum("C1", 0)))
+    env.set("C1", 0, A)
+    assert np.max(np.abs(env.corner_spectrum("C1", 0) - good / np.linalg.norm(good))) < 3e-13
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 400), (31, 33, 15), (32, 32, 16), (33, 31, 17), (32, 700, 400),
                                    (700, 32, 401), (33, 33, 400), (1024, 2048, 31), (1025, 2047, 33),
                                    (2500, 128, 128), (128, 128, 400), (32, 32, 8191), (32, 32, 8192),
