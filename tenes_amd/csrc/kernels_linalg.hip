@@ -659,12 +659,16 @@ __device__ __forceinline__ double sum16(double v) {
 // recomputed in the update, pick the next pivot in every wave).  At 40 x 40 it
 // costs 76 us, and Jacobi and replay fall from 586 + 219 to 189 + 18 us.
 constexpr int kQrpThreads = 1024;
+// smallest squared norm of a remainder that is still reflected (the matrix
+// scaled to a largest entry in [1, 2))
+constexpr double kQrpNull = 1e-280;
 
 __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int m, int n,
                                                           double *Wg, double *Qg) {
   extern __shared__ double S[];  // m rows of n, padded to ld
   __shared__ double s_nrm[2][kMaxDim];  // squared norm of the rest, -1: used
   __shared__ double s_tau[kMaxDim], s_head[kMaxDim], s_alpha[kMaxDim];
+  __shared__ double s_big[kQrpThreads / 64];
   __shared__ int s_piv[kMaxDim], s_pos[kMaxDim];
   constexpr int NG = kQrpThreads / 16;
   const int ld = n | 1;
@@ -675,12 +679,16 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
   double *W = Wg + (int64_t)blockIdx.x * m * r;
   double *Q = Qg ? Qg + (int64_t)blockIdx.x * n * r : nullptr;
   bool finite = true;
+  double big = 0.0;
   for (int e = tid; e < m * n; e += kQrpThreads) {
     const int j = e / n;
     const double v = A[e];
     finite = finite && fabs(v) <= DBL_MAX;
+    big = fmax(big, fabs(v));
     S[j * ld + (e - j * n)] = v;
   }
+  for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+  if (lane == 0) s_big[tid >> 6] = big;
   if (tid < m) s_pos[tid] = r;
   // a NaN or infinite entry: every value and vector of this matrix is NaN
   // (below, a NaN norm would be taken for the norm of a zero row)
@@ -690,6 +698,17 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
     for (int e = tid; Q && e < n * r; e += kQrpThreads) Q[e] = nan;
     return;
   }
+  // scaled by a power of two (exact) to a largest entry in [1, 2), as in
+  // jacobi_kernel: the squared norms do not overflow, and vanish only for rows
+  // 1e-154 times the largest entry
+  for (int w = 0; w < kQrpThreads / 64; ++w) big = fmax(big, s_big[w]);
+  const int ex = big > 0.0 ? __builtin_amdgcn_frexp_exp(big) - 1 : 0;
+  for (int e = tid; e < m * n; e += kQrpThreads) {  // the elements this thread stored
+    const int j = e / n;
+    double &x = S[j * ld + (e - j * n)];
+    x = __builtin_amdgcn_ldexp(x, -ex);
+  }
+  __syncthreads();
   for (int j = grp; j < m; j += NG) {
     double acc = 0.0;
     for (int i = gl; i < n; i += 16) acc = fma(S[j * ld + i], S[j * ld + i], acc);
@@ -697,6 +716,7 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
     if (gl == 0) s_nrm[0][j] = acc;
   }
   __syncthreads();
+  int done = 0;  // reflections made
   for (int k = 0; k < r; ++k) {
     const double *cur = s_nrm[k & 1];
     double *next = s_nrm[(k + 1) & 1];
@@ -716,16 +736,18 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
       }
     }
     bj = __builtin_amdgcn_readfirstlane(bj);
+    // What remains is zero, or too small for 1 / (squared norm): no more
+    // reflections.  The rows not used keep their entries (past column r they
+    // are dropped, 1e-140 of the largest).
+    if (!(best > kQrpNull)) break;
+    done = k + 1;
     // Householder vector of its elements k..n-1 (in place; the head apart)
     const double *v = S + bj * ld;
     const double bk = v[k];
-    double al = 0.0, tau = 0.0, head = 0.0;
-    if (best > 0.0) {
-      const double nb = sqrt(best);
-      al = bk > 0.0 ? -nb : nb;
-      head = bk - al;
-      tau = 1.0 / (best + fabs(bk) * nb);
-    }
+    const double nb = sqrt(best);
+    const double al = bk > 0.0 ? -nb : nb;
+    const double head = bk - al;
+    const double tau = 1.0 / (best + fabs(bk) * nb);
     if (tid == 0) {
       s_tau[k] = tau;
       s_head[k] = head;
@@ -765,7 +787,8 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
   for (int e = tid; e < m * r; e += kQrpThreads) {
     const int c = e / m, j = e - c * m;
     const int pos = s_pos[j];
-    W[e] = c < pos ? S[j * ld + c] : (c == pos ? s_alpha[c] : 0.0);
+    W[e] = c < pos ? __builtin_amdgcn_ldexp(S[j * ld + c], ex)
+                   : (c == pos ? __builtin_amdgcn_ldexp(s_alpha[c], ex) : 0.0);
   }
   if (!Q) return;
   // Q = H_0 ... H_{r-1} (unit columns): column c on one group, in registers
@@ -773,7 +796,7 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
     double q[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) q[u] = gl + 16 * u == c ? 1.0 : 0.0;
-    for (int k = c; k >= 0; --k) {
+    for (int k = min(c, done - 1); k >= 0; --k) {
       const double *v = S + s_piv[k] * ld;
       const double head = s_head[k];
       double vv[8], dot = 0.0;

@@ -361,6 +361,48 @@ def test_exact_svd_reports_non_finite_input(gpu_ctx, m, n, at, bad):
     assert np.max(np.abs(env.corner_spectrum("C1", 0) - good / np.linalg.norm(good))) < 3e-13
 
 
+def _graded(rng, m, n, scale, decades=10):
+    """m x n with singular values over `decades` decades below `scale`."""
+    k = min(m, n)
+    q1, _ = np.linalg.qr(rng.standard_normal((m, k)))
+    q2, _ = np.linalg.qr(rng.standard_normal((n, k)))
+    return (q1 * np.logspace(0, -decades, k)) @ q2.T * scale
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (5, 3), (3, 5), (40, 40), (33, 64), (64, 33), (128, 128)])
+@pytest.mark.parametrize("scale", [1e-290, 1e-200, 1e200, 1e290])
+def test_exact_svd_scale(gpu_ctx, m, n, scale):
+    """Entries whose squares overflow or vanish: the exact path is scaled by
+    powers of two, so the errors relative to the largest value are those of
+    test_jacobi_svd_slot_edges (3e-13)."""
+    A = _graded(np.random.default_rng(m + 2 * n), m, n, scale)
+    k = min(m, n)
+    U, s, V = ta.svd_top(gpu_ctx.tensor(A), k)
+    U, V = U.numpy(), V.numpy()
+    ref = np.linalg.svd(A / scale, compute_uv=False)
+    assert np.max(np.abs(s / scale - ref)) < 3e-13
+    assert np.max(np.abs((U * (s / scale)) @ V.T - A / scale)) < 3e-13
+    assert np.max(np.abs(V.T @ V - np.eye(k))) < 3e-13
+    assert np.max(np.abs(U.T @ U - np.eye(k))) < 3e-13
+
+
+@pytest.mark.parametrize("m,n", [(2, 2), (5, 5), (4, 9), (9, 4), (64, 64)])
+@pytest.mark.parametrize("tiny", [1e-130, 1e-145, 1e-155, 1e-157, 1e-162, 1e-200, 0.0])
+def test_exact_svd_decoupled_small_entry(gpu_ctx, m, n, tiny):
+    """A remainder of the QR whose squared norm is denormal or zero beside an
+    entry of 1 (a decoupled index): nothing overflows in 1 / (squared norm),
+    the factors stay finite and orthonormal, and 1e-130 keeps its value."""
+    A = np.zeros((m, n))
+    A[0, 0], A[-1, -1] = 1.0, tiny
+    U, s, V = ta.svd_top(gpu_ctx.tensor(A), 2)
+    U, V = U.numpy(), V.numpy()
+    assert s[0] == 1.0 and 0.0 <= s[1] <= 1.001 * tiny
+    if tiny == 1e-130:
+        assert abs(s[1] - tiny) < 1e-12 * tiny
+    assert np.all(np.isfinite(U)) and np.max(np.abs(V.T @ V - np.eye(2))) < 1e-15
+    assert abs(abs(U[0, 0]) - 1.0) < 1e-15 and abs(abs(V[0, 0]) - 1.0) < 1e-15
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 400), (31, 33, 15), (32, 32, 16), (33, 31, 17), (32, 700, 400),
                                    (700, 32, 401), (33, 33, 400), (1024, 2048, 31), (1025, 2047, 33),
                                    (2500, 128, 128), (128, 128, 400), (32, 32, 8191), (32, 32, 8192),
