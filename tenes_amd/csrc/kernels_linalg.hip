@@ -1014,8 +1014,30 @@ __global__ __launch_bounds__(1024) void jacobi_big_kernel(
   double *W = Wg + (int64_t)b * m * p;
   const int pe = p + (p & 1);
   const int tid = threadIdx.x;
-  double fro = 0.0;
-  for (int i = tid; i < m * p; i += blockDim.x) fro += W[i] * W[i];
+  // A largest entry outside [2^-100, 2^100] is scaled by a power of two
+  // (exact), as in jacobi_kernel; between them the squared norms down to the
+  // 1e-60 of s_tiny and their products with tol^2 stay in range, and the
+  // pass over global memory is saved.
+  double fro = 0.0, big = 0.0;
+  for (int i = tid; i < m * p; i += blockDim.x) {
+    fro += W[i] * W[i];
+    big = fmax(big, fabs(W[i]));
+  }
+  for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+  if ((tid & 63) == 0) s_off[tid >> 6] = big;
+  __syncthreads();
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) big = fmax(big, s_off[w]);
+  __syncthreads();
+  int ex = big > 0.0 && big <= DBL_MAX ? __builtin_amdgcn_frexp_exp(big) - 1 : 0;
+  if (ex >= -100 && ex <= 100) ex = 0;
+  if (ex != 0) {
+    fro = 0.0;
+    for (int i = tid; i < m * p; i += blockDim.x) {
+      const double v = __builtin_amdgcn_ldexp(W[i], -ex);
+      W[i] = v;
+      fro += v * v;
+    }
+  }
   for (int o = 32; o > 0; o >>= 1) fro += __shfl_xor(fro, o, 64);
   if ((tid & 63) == 0) s_off[tid >> 6] = fro;
   __syncthreads();
@@ -1093,7 +1115,11 @@ __global__ __launch_bounds__(1024) void jacobi_big_kernel(
     double acc = 0.0;
     const double *wc = W + (int64_t)jc * m;
     for (int r = 0; r < m; ++r) acc += wc[r] * wc[r];
-    sigma[(int64_t)b * p + jc] = sqrt(acc);
+    sigma[(int64_t)b * p + jc] = __builtin_amdgcn_ldexp(sqrt(acc), ex);
+  }
+  if (ex != 0) {
+    __syncthreads();  // the norms above read the columns
+    for (int i = tid; i < m * p; i += blockDim.x) W[i] = __builtin_amdgcn_ldexp(W[i], ex);
   }
   if (tid == 0 && nsteps) nsteps[b] = steps;
 }

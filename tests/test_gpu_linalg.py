@@ -386,6 +386,22 @@ def test_exact_svd_scale(gpu_ctx, m, n, scale):
     assert np.max(np.abs(U.T @ U - np.eye(k))) < 3e-13
 
 
+@pytest.mark.parametrize("m,n", [(129, 129), (160, 130), (130, 160), (256, 256), (20, 200)])
+@pytest.mark.parametrize("power", [-460, -300, -101, -99, 99, 101, 300, 460])
+def test_large_corner_spectrum_scale(gpu_ctx, m, n, power):
+    """Spectra of corners above 128 (the Jacobi in global memory), far from
+    unit scale and on both sides of its scaling limit of 2^100.  A power of
+    two changes no rounding while nothing overflows or vanishes, so the
+    normalised spectrum has the bits of the unscaled matrix's.  (The host's
+    normalisation squares the values: a corner stays within 2^500.)"""
+    A = _graded(np.random.default_rng(m + 2 * n), m, n, 1.0)
+    env = ta.Environment(gpu_ctx, 1, 1)
+    env.set("C1", 0, A)
+    ref = env.corner_spectrum("C1", 0)
+    env.set("C1", 0, np.ldexp(A, power))
+    assert np.array_equal(env.corner_spectrum("C1", 0), ref)
+
+
 @pytest.mark.parametrize("m,n", [(2, 2), (5, 5), (4, 9), (9, 4), (64, 64)])
 @pytest.mark.parametrize("tiny", [1e-130, 1e-145, 1e-155, 1e-157, 1e-162, 1e-200, 0.0])
 def test_exact_svd_decoupled_small_entry(gpu_ctx, m, n, tiny):
