@@ -91,9 +91,9 @@ int tenes_ctx_set_fp32_contractions(tenes_ctx *ctx, int on);
 int tenes_ctx_set_fused_site(tenes_ctx *ctx, int on);
 /* GEMM autotuning of a context (on != 0): the first contraction of every
  * plan (operand shapes and legs) with at least 1e8 flops times each candidate
- * launch shape of the gather-GEMM (64 or 128 tiles, split-K counts) twice on
- * the context's stream, synchronising, and keeps the fastest for that plan;
- * later contractions of the plan launch it directly.  Results change only at
+ * launch shape of the gather-GEMM (32, 64 or 128 tiles, split-K counts) twice
+ * on the context's stream, synchronising, and keeps the fastest for that plan
+ * and contraction mode; later contractions of the plan launch it directly.  Results change only at
  * rounding (split-K sums in another order).  Off by default.  No
  * counterpart in the reference. */
 int tenes_ctx_set_autotune(tenes_ctx *ctx, int on);

@@ -44,18 +44,19 @@ struct GemmArgs {
   bool bf16x3 = false;
 };
 
-// A GEMM launch shape: square output tile (64 or 128) and the number of K
-// splits; bm = 0 selects the built-in heuristic.
+// A GEMM launch shape: square output tile (64, 128 or, in FP64, 32) and the
+// number of K splits; bm = 0 selects the built-in heuristic (gemm_plan.hpp).
 struct GemmPlan {
   int bm = 0;
   int splits = 0;
 };
-// Launch shapes worth timing for (M, N, K), the heuristic's first.
 // The stream-K launch of an M x N x K FP64 product (GemmPlan{128, 0}) exists:
 // 128 x 128 tiles leaving at least half a round of 512 workgroups after the
 // whole rounds, and K of at least 64 tiles of 16.
 bool gemm_stream_k(int M, int N, int K);
-std::vector<GemmPlan> gemm_candidates(int M, int N, int K);
+// Launch shapes worth timing for (M, N, K) in FP64 or in the FP32 and split
+// bf16 modes, the heuristic's first.
+std::vector<GemmPlan> gemm_candidates(int M, int N, int K, bool f64);
 // Scratch needed for split-K on the given shape (bytes, 0 if none).
 size_t gemm_workspace_bytes(int M, int N, int K, const GemmPlan *plan = nullptr,
                             bool f64 = true);

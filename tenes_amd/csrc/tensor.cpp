@@ -880,14 +880,16 @@ static void contract_into(Context &ctx, const ContractPlan &p, const Tensor &A, 
   const double flops = 2.0 * p.M * (double)p.N * p.K;
   // autotuning (C = A B overwrites C, so every candidate leaves a valid
   // result): time each launch shape twice on this stream, keep the fastest
-  if (ctx.autotune() && !ctx.capturing() && beta == 0.0 && p.tuned_bm == 0 &&
+  const bool f64 = !g.fp32 && !g.bf16x3;
+  kern::GemmPlan &tuned = p.tuned[ctx.contraction_mode()];
+  if (ctx.autotune() && !ctx.capturing() && beta == 0.0 && tuned.bm == 0 &&
       flops >= Context::kAutotuneFlops) {
     hipEvent_t e0, e1;
     TN_HIP_CHECK(hipEventCreate(&e0));
     TN_HIP_CHECK(hipEventCreate(&e1));
     float best = 0.0f;
-    for (const kern::GemmPlan &c : kern::gemm_candidates(p.M, p.N, p.K)) {
-      const size_t cws = kern::gemm_workspace_bytes(p.M, p.N, p.K, &c);
+    for (const kern::GemmPlan &c : kern::gemm_candidates(p.M, p.N, p.K, f64)) {
+      const size_t cws = kern::gemm_workspace_bytes(p.M, p.N, p.K, &c, f64);
       void *cw = cws ? ctx.workspace(cws) : nullptr;
       TN_HIP_CHECK(hipEventRecord(e0, ctx.stream()));
       kern::gemm_f64(g, cw, cws, ctx.stream(), &c);
@@ -896,21 +898,19 @@ static void contract_into(Context &ctx, const ContractPlan &p, const Tensor &A, 
       TN_HIP_CHECK(hipEventSynchronize(e1));
       float ms = 0.0f;
       TN_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-      if (p.tuned_bm == 0 || ms < best) {
+      if (tuned.bm == 0 || ms < best) {
         best = ms;
-        p.tuned_bm = c.bm;
-        p.tuned_splits = c.splits;
+        tuned = c;
       }
     }
     TN_HIP_CHECK(hipEventDestroy(e0));
     TN_HIP_CHECK(hipEventDestroy(e1));
   }
-  kern::GemmPlan tuned{p.tuned_bm, p.tuned_splits};
-  const kern::GemmPlan *plan = p.tuned_bm ? &tuned : nullptr;
+  const kern::GemmPlan *plan = tuned.bm ? &tuned : nullptr;
   static const kern::GemmPlan kStreamK{128, 0};
-  if (!plan && ctx.stream_k() && !g.fp32 && !g.bf16x3 && kern::gemm_stream_k(p.M, p.N, p.K))
+  if (!plan && ctx.stream_k() && f64 && kern::gemm_stream_k(p.M, p.N, p.K))
     plan = &kStreamK;
-  const size_t ws = kern::gemm_workspace_bytes(p.M, p.N, p.K, plan, !g.fp32 && !g.bf16x3);
+  const size_t ws = kern::gemm_workspace_bytes(p.M, p.N, p.K, plan, f64);
   void *w = ws ? ctx.workspace(ws) : nullptr;
   if (ctx.profiling()) {
     hipEvent_t a;

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "kernels.hpp"
 
 namespace tn {
 
@@ -111,8 +112,9 @@ struct ContractPlan {
   int a_m_off, a_k_off, b_k_off, b_n_off, c_m_off, c_n_off;
   bool a_mfast = false, b_nfast = false;
   int a_m_stride = 0, a_k_stride = 0, b_k_stride = 0, b_n_stride = 0;
-  // GEMM launch shape picked by the autotuner (bm = 0: not tuned yet)
-  mutable int tuned_bm = 0, tuned_splits = 0;
+  // GEMM launch shapes picked by the autotuner, one for each contraction
+  // mode (bm = 0: not tuned yet): their kernels differ
+  mutable kern::GemmPlan tuned[3];
 };
 
 class Context {

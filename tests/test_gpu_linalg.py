@@ -250,6 +250,27 @@ def test_gemm_autotune():
     ctx.close()
 
 
+def test_gemm_autotune_each_mode():
+    """One plan tuned in FP64, FP32 and split bf16 in turn (1000 x 400 x 400:
+    32 x 32 tiles in FP64, split K in the others): every mode keeps its own
+    launch shape, and its results stay within its own bound: 1e-12, the FP32
+    summation bound, and three times the 2^-16 of a dropped low x low product
+    beside it."""
+    ctx = ta.Context(0, seed=5)
+    ctx.set_autotune(True)
+    rng = np.random.default_rng(10)
+    A, B = rng.standard_normal((1000, 400)), rng.standard_normal((400, 400))
+    ref, mag = A @ B, np.abs(A) @ np.abs(B)
+    a, b = ctx.tensor(A), ctx.tensor(B)
+    fp32 = 402 * 2.0 ** -24 * mag
+    for mode in (0, 1, 2, 0, 2, 1):
+        ctx.set_contraction_mode(mode)
+        C = ta.tensordot(a, b, [1], [0]).numpy()
+        bound = (1e-12 * np.max(np.abs(ref)), fp32, fp32 + 3 * 2.0 ** -16 * mag)[mode]
+        assert np.all(np.abs(C - ref) <= bound), mode
+    ctx.close()
+
+
 def test_autotuned_ctm_matches_oracle():
     """A CTM run with autotuning on (fresh context): energy and Sz against the
     oracle to 1e-10, as without it."""
