@@ -14,6 +14,7 @@ namespace kern {
 
 constexpr int BK = 16;         // depth of a K tile
 constexpr int kSkRanks = 512;  // stream-K grid: two workgroups per CU
+constexpr int kMaxTileRows = 65535;  // workgroups of a launch in y (rows of tiles)
 
 struct Plan {
   int BM, BN, splits, kps;
@@ -73,10 +74,11 @@ inline Plan choose(int M, int N, int K, bool f64) {
   // columns waste less of the tile.  Back to back, with the host's 8.4 us per
   // call as the floor: 2500 x 128 x 128 13.2 to 8.1 us, 333 x 128 x 333 12.0
   // to 9.7, 1024 x 1024 x 64 10.4 to 8.4.  Above 2048 tiles the 64 x 64 grid
-  // fills the chip and moves less through L2.
+  // fills the chip and moves less through L2.  (A thin output of more than
+  // 65535 rows of 32 tiles is past the grid's limit.)
   const int64_t tiles32 = (int64_t)ceil_div(M, 32) * ceil_div(N, 32);
   const bool thin = M <= 32 || N <= 32;
-  if (f64 && K <= 400 && (thin || tiles32 <= 2048)) {
+  if (f64 && K <= 400 && (thin || tiles32 <= 2048) && ceil_div(M, 32) <= kMaxTileRows) {
     p.BM = p.BN = 32;
     p.splits = 1;
     p.kps = ceil_div(K, BK) * BK;

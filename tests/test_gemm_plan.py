@@ -72,3 +72,15 @@ def test_splits_cover_k(lib, f64):
             bm, splits, kps, _ = plan(lib, M, N, K, f64, c)
             assert bm in (32, 64, 128) and kps % 16 == 0
             assert (splits - 1) * kps < K <= splits * kps, (M, N, K, c)
+
+
+@pytest.mark.parametrize("M", [2097120, 2097121, 4194240])
+@pytest.mark.parametrize("N", [1, 32, 33])
+@pytest.mark.parametrize("K", [1, 400, 8192])
+def test_tall_products_stay_in_the_grid(lib, M, N, K):
+    """65535 workgroups in y: M up to 64 x 65535 has a launch, as it had with
+    64 x 64 tiles alone, tuned or not."""
+    for f64 in (True, False):
+        bm = plan(lib, M, N, K, f64)[0]
+        assert -(-M // bm) <= 65535, (bm, f64)
+        assert all(c[0] != 32 for c in candidates(lib, M, N, K, f64)) or M <= 2097120
