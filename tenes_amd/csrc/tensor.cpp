@@ -253,6 +253,9 @@ void Context::spread_lanes() {
   const int n = (int)lanes_.size() - 1;
   kern::lane_probe(lanes_[1].scal, 0, lanes_[1].s);  // load the kernel
   TN_HIP_CHECK(hipStreamSynchronize(lanes_[1].s));
+  // work queued on the main stream would hold back the lanes that share its
+  // hardware queue, and they would be taken for overlapping none
+  TN_HIP_CHECK(hipStreamSynchronize(lanes_[0].s));
   for (int i = 1; i <= n; ++i) kern::lane_probe(lanes_[i].scal, kern::kProbeTicks, lanes_[i].s);
   std::vector<std::array<int64_t, 2>> t(n + 1);
   for (int i = 1; i <= n; ++i) {
