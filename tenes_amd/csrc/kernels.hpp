@@ -207,11 +207,11 @@ void jacobi_svd(double *W, int m, int p, int batch, double tol,
 // written).
 void jacobi_accumulate(const double *rot, const int *nsteps, int p, double *J,
                        hipStream_t s, const double *J0 = nullptr, int rows = 0);
-// Preconditioner of jacobi_svd for m, n <= 128 (a batch of m x n row-major
-// matrices): A = W Q^T from the row-pivoted QR of A^T, W (m x r column-major,
+// Preconditioner of jacobi_svd for an m x n row-major matrix, m, n <= 128:
+// A = W Q^T from the row-pivoted QR of A^T, W (m x r column-major,
 // r = min(m, n)) with columns of falling length, Q (n x r row-major)
-// orthonormal columns, or nullptr.
-void qrp(const double *A, int m, int n, int batch, double *W, double *Q, hipStream_t s);
+// orthonormal columns.
+void qrp(const double *A, int m, int n, double *W, double *Q, hipStream_t s);
 // sorted[b][r] = sigma[b][perm[b][r]], descending (ties keep index order, NaN
 // last: perm is a permutation whatever the values).
 void sort_desc(const double *sigma, int p, int batch, double *sorted,

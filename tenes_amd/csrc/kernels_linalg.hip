@@ -647,7 +647,7 @@ __device__ __forceinline__ double sum16(double v) {
 }
 
 // Pivoted Householder QR of A^T (A: m x n row-major, m, n <= 128, one
-// workgroup per matrix) as the preconditioner of the one-sided Jacobi SVD:
+// workgroup) as the preconditioner of the one-sided Jacobi SVD:
 //   A = W Q^T, Q (n x r) orthonormal, W = A Q (m x r), r = min(m, n).
 // W is lower triangular up to the order of its rows, with columns of falling
 // length, and its columns are close to orthogonal: the Jacobi needs 5 to 7
@@ -663,8 +663,8 @@ constexpr int kQrpThreads = 1024;
 // scaled to a largest entry in [1, 2))
 constexpr double kQrpNull = 1e-280;
 
-__global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int m, int n,
-                                                          double *Wg, double *Qg) {
+__global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *A, int m, int n,
+                                                          double *W, double *Q) {
   extern __shared__ double S[];  // m rows of n, padded to ld
   __shared__ double s_nrm[2][kMaxDim];  // squared norm of the rest, -1: used
   __shared__ double s_tau[kMaxDim], s_head[kMaxDim], s_alpha[kMaxDim];
@@ -675,9 +675,6 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
   const int r = min(m, n);
   const int tid = threadIdx.x, lane = tid & 63;
   const int grp = tid >> 4, gl = tid & 15;
-  const double *A = Ag + (int64_t)blockIdx.x * m * n;
-  double *W = Wg + (int64_t)blockIdx.x * m * r;
-  double *Q = Qg ? Qg + (int64_t)blockIdx.x * n * r : nullptr;
   bool finite = true;
   double big = 0.0;
   for (int e = tid; e < m * n; e += kQrpThreads) {
@@ -695,7 +692,7 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
   if (__syncthreads_or(!finite)) {
     const double nan = __builtin_nan("");
     for (int e = tid; e < m * r; e += kQrpThreads) W[e] = nan;
-    for (int e = tid; Q && e < n * r; e += kQrpThreads) Q[e] = nan;
+    for (int e = tid; e < n * r; e += kQrpThreads) Q[e] = nan;
     return;
   }
   // scaled by a power of two (exact) to a largest entry in [1, 2), as in
@@ -790,7 +787,6 @@ __global__ __launch_bounds__(kQrpThreads) void qrp_kernel(const double *Ag, int 
     W[e] = c < pos ? __builtin_amdgcn_ldexp(S[j * ld + c], ex)
                    : (c == pos ? __builtin_amdgcn_ldexp(s_alpha[c], ex) : 0.0);
   }
-  if (!Q) return;
   // Q = H_0 ... H_{r-1} (unit columns): column c on one group, in registers
   for (int c = grp; c < r; c += NG) {
     double q[8];
@@ -1403,11 +1399,10 @@ void jacobi_svd(double *W, int m, int p, int batch, double tol,
   TN_HIP_CHECK(hipGetLastError());
 }
 
-void qrp(const double *A, int m, int n, int batch, double *W, double *Q, hipStream_t s) {
+void qrp(const double *A, int m, int n, double *W, double *Q, hipStream_t s) {
   TN_REQUIRE(m >= 1 && n >= 1 && m <= kMaxDim && n <= kMaxDim, "qrp: dimension out of range");
-  if (batch <= 0) return;
   const size_t lds = (size_t)m * (n | 1) * sizeof(double);
-  hipLaunchKernelGGL(qrp_kernel, dim3(batch), dim3(kQrpThreads), lds, s, A, m, n, W, Q);
+  hipLaunchKernelGGL(qrp_kernel, dim3(1), dim3(kQrpThreads), lds, s, A, m, n, W, Q);
   TN_HIP_CHECK(hipGetLastError());
 }
 

@@ -306,7 +306,7 @@ SvdPending svd_top_begin_impl(Context &ctx, const Tensor *Ap, const LinearOp *op
   } else {
     const int r = std::min(rows, cols);
     Tensor W = empty(ctx, Shape{r, rows}), Q0 = empty(ctx, Shape{cols, r});
-    kern::qrp(X.data(), rows, cols, 1, W.data(), Q0.data(), s);
+    kern::qrp(X.data(), rows, cols, W.data(), Q0.data(), s);
     run_jacobi(ctx, W, rows, r, true, opt, jo, Q0);
     cols = r;
   }
@@ -380,23 +380,23 @@ Tensor svd_values_batched(Context &ctx, const std::vector<Tensor> &mats) {
              "svd_values_batched: matrices larger than 256 x 256");
   const int b = (int)mats.size();
   hipStream_t s = ctx.stream();
-  // Jacobi acts on the columns of the stored column-major matrix.  Up to 128
-  // it is preconditioned (kern::qrp, which leaves min(m, n) columns of length
-  // m); above, the shorter side is the column length: for m >= n store X
-  // column-major, else orthogonalise the columns of X^T.
-  const bool small = m <= kJac && n <= kJac;
-  const bool tr = !small && m < n;
-  const int rows = tr ? n : m, cols = small ? std::min(m, n) : tr ? m : n;
+  // Jacobi acts on the columns of the stored column-major matrix.  Use the
+  // shorter side as the column length: for m >= n store X column-major.  No
+  // preconditioner (kern::qrp): corners are nearly diagonal and take few sweeps
+  // as they are, and without a right factor to replay those are all it saves
+  // (spectra of corners from D=2..5 runs, chi = 8, 27, 45, 64, 100: 50, 97, 150,
+  // 474, 1189 us without, 64, 157, 218, 554, 1383 us with it).
+  const bool tr = m < n;  // then orthogonalise the columns of X^T
+  const int rows = tr ? n : m, cols = tr ? m : n;
   Tensor W = empty(ctx, Shape{b, cols, rows});
-  Tensor in = small ? empty(ctx, Shape{b, m, n}) : W;
   for (int i = 0; i < b; ++i) {
     TN_REQUIRE(mats[i].shape == mats[0].shape,
                "svd_values_batched: shape mismatch in batch");
-    Tensor src = small || tr ? mats[i] : transpose(mats[i], Axes{1, 0});
-    TN_HIP_CHECK(hipMemcpyAsync(in.data() + (int64_t)i * m * n, src.data(),
-                                sizeof(double) * m * n, hipMemcpyDeviceToDevice, s));
+    Tensor src = tr ? mats[i] : transpose(mats[i], Axes{1, 0});
+    TN_HIP_CHECK(hipMemcpyAsync(W.data() + (int64_t)i * rows * cols,
+                                src.data(), sizeof(double) * rows * cols,
+                                hipMemcpyDeviceToDevice, s));
   }
-  if (small) kern::qrp(in.data(), m, n, b, W.data(), nullptr, s);
   Tensor sigma = empty(ctx, Shape{b, cols});
   SvdOptions opt;
   kern::jacobi_svd(W.data(), rows, cols, b, jacobi_tol_for(opt, rows),

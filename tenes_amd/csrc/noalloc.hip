@@ -104,7 +104,7 @@ void svd_small(int device, hipStream_t s, const double *A, int m, int n, int k,
   // A = W J^T preconditioned, then the Jacobi on the r columns of W and its
   // rotations replayed on J in place, as svd_top does on this path
   const int r = std::min(m, n);
-  kern::qrp(A, m, n, 1, W, J, s);
+  kern::qrp(A, m, n, W, J, s);
   const double tol = std::sqrt((double)m) * 2.220446049250313e-16;
   kern::jacobi_svd(W, m, r, 1, tol, kSweeps, sigma, rot, nsteps, s);
   kern::sort_desc(sigma, r, 1, sorted, perm, s);
