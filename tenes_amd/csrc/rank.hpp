@@ -1,16 +1,21 @@
-// The order of singular values: descending, NaN after every number, equal
-// ones by index.  A total order, so the ranks of any p values are a
-// permutation of 0..p-1 (every comparison with NaN is false: ranks counted
-// with > and == alone would repeat, and the permutation that gathers the
-// singular vectors would keep unwritten entries).
+// The order of singular values: descending by rank_key, equal keys by index.
+// A NaN gets the lowest key, so it comes after every number and the keys are
+// totally ordered: the ranks of any p values are a permutation of 0..p-1.
+// (Every comparison with NaN is false: ranks counted on the values themselves
+// would repeat, and the permutation that gathers the singular vectors would
+// keep unwritten entries.)
 #pragma once
+
+#include <limits>
 
 namespace tn {
 
-// whether value u at index k comes before value v at index j
+constexpr double rank_key(double v) {
+  return v == v ? v : -std::numeric_limits<double>::infinity();
+}
+
+// whether the value of key u at index k comes before that of key v at index j
 constexpr bool ranks_before(double u, int k, double v, int j) {
-  const bool un = u != u, vn = v != v;
-  if (un || vn) return un == vn ? k < j : vn;
   return u > v || (u == v && k < j);
 }
 

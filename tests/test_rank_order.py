@@ -15,7 +15,7 @@ CSRC = Path(__file__).resolve().parents[1] / "tenes_amd" / "csrc"
 def before(tmp_path_factory):
     d = tmp_path_factory.mktemp("rank")
     (d / "r.cpp").write_text('#include "rank.hpp"\nextern "C" int before(double u, int k, double v, int j) '
-                             "{ return tn::ranks_before(u, k, v, j); }\n")
+                             "{ return tn::ranks_before(tn::rank_key(u), k, tn::rank_key(v), j); }\n")
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(d / "r.cpp"), "-o", str(d / "r.so")],
                    check=True)
     f = ctypes.CDLL(str(d / "r.so")).before
