@@ -382,6 +382,50 @@ def test_exact_svd_reports_non_finite_input(gpu_ctx, m, n, at, bad):
     assert np.max(np.abs(env.corner_spectrum("C1", 0) - good / np.linalg.norm(good))) < 3e-13
 
 
+_I = np.arange(400)
+_SPECTRA = {
+    "exponential": np.exp(-0.2 * _I),
+    "flat_exponential": np.exp(-0.1 * _I),
+    "algebraic": (1.0 + _I) ** -6.0,
+    "step_1e-9": np.where(_I < 10, 1.0, 1e-9) * np.exp(-0.1 * _I),
+    "step_1e-5": np.where(_I < 60, 1.0, 1e-5) * np.exp(-0.1 * _I),
+    "two_steps": np.where(_I < 20, 1.0, np.where(_I < 60, 1e-6, 1e-11)) * np.exp(-0.1 * _I),
+    "degenerate": np.exp(-0.2 * (_I // 8 * 8)),
+    "flat_rank_100": np.where(_I < 100, 1.0, 0.0),
+    "rank_30": np.where(_I < 30, np.exp(-0.3 * _I), 0.0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(_SPECTRA))
+@pytest.mark.parametrize("q", [1, 2, 8])
+def test_range_finder_spectra(gpu_ctx, name, q):
+    """The 128-wide range finder from a Gaussian block (two shifted
+    orthonormalisations in the first iteration, plain ones after) on 400 x 400
+    matrices of nine kinds of spectra, against LAPACK: values, residuals of the
+    triplets and orthogonality of the directions above the plain passes'
+    pivot floor.  Tolerance, of the largest value: the subspace error
+    (s_129 / s_k)^(2q+1) times s_k (k = 60; measured against the spectrum
+    itself, times 100 for the Gaussian block's constant) and 3e-13 for the
+    arithmetic (128 eps times ten)."""
+    rng = np.random.default_rng(len(name) + q)
+    sv, k = _SPECTRA[name], 60
+    q1, _ = np.linalg.qr(rng.standard_normal((400, 400)))
+    q2, _ = np.linalg.qr(rng.standard_normal((400, 400)))
+    A = (q1 * sv) @ q2.T
+    U, s, V = ta.svd_top(gpu_ctx.tensor(A), k, power_iters=q)
+    U, V = U.numpy(), V.numpy()
+    err = 100.0 * sv[k - 1] * (sv[128] / sv[k - 1]) ** (2 * q + 1) if sv[k - 1] > 0.0 else 0.0
+    tol = 3e-13 + err / sv[0]
+    assert np.max(np.abs(s - sv[:k])) < tol * sv[0]
+    r = int(np.sum(s > 1e-12 * s[0]))
+    assert r == int(np.sum(sv[:k] > 1e-12))
+    assert np.max(np.abs(A @ V[:, :r] - U[:, :r] * s[:r])) < tol * sv[0]
+    # exact for U in the range found: only the arithmetic
+    assert np.max(np.abs(A.T @ U[:, :r] - V[:, :r] * s[:r])) < 3e-13 * sv[0]
+    for X in (U, V):
+        assert np.max(np.abs(X[:, :r].T @ X[:, :r] - np.eye(r))) < 3e-13
+
+
 def _graded(rng, m, n, scale, decades=10):
     """m x n with singular values over `decades` decades below `scale`."""
     k = min(m, n)
