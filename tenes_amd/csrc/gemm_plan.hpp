@@ -98,7 +98,8 @@ inline Plan choose(int M, int N, int K, bool f64) {
     // a few tiles and a very long K (density matrices and their gradients,
     // 32 x 16 x 131072): the operands stream from HBM once, so as many
     // workgroups as 1024 over the tiles, at least eight K tiles each; 64
-    // splits left three quarters of the CUs idle (165 us, 40 us now)
+    // splits left three quarters of the CUs idle (133 to 143 us by layout,
+    // 20 us now, the reduction included)
     p.splits = std::min(K / (8 * BK), 1024 / (int)tiles);
   } else if (tiles < 128 && K >= 4 * BK * 2) {
     const int maxs = std::max(1, K / (4 * BK));

@@ -651,13 +651,14 @@ __device__ __forceinline__ double sum16(double v) {
 //   A = W Q^T, Q (n x r) orthonormal, W = A Q (m x r), r = min(m, n).
 // W is lower triangular up to the order of its rows, with columns of falling
 // length, and its columns are close to orthogonal: the Jacobi needs 5 to 7
-// sweeps on it where the matrices of the small environments (40 x 40, graded
-// over 11 decades) took 15 to 17, and r columns instead of n.  A row of A is a
+// sweeps on it where the projector matrices of a D=2, chi=10 run (40 x 40,
+// graded over 11 decades) took 15 to 17, and r columns instead of n.  A row of A is a
 // column of A^T, so the pivot is the longest remaining row, and no row is
 // moved: used rows keep their Householder vector.  64 groups of 16 lanes, a
 // row per group; one barrier per step (the norms of the rows' remainders,
-// recomputed in the update, pick the next pivot in every wave).  At 40 x 40 it
-// costs 76 us, and Jacobi and replay fall from 586 + 219 to 189 + 18 us.
+// recomputed in the update, pick the next pivot in every wave).  On those 40 x 40
+// matrices it costs 90 us, and Jacobi and replay fall from 720 + 219 to
+// 228 + 18 us.
 constexpr int kQrpThreads = 1024;
 // smallest squared norm of a remainder that is still reflected (the matrix
 // scaled to a largest entry in [1, 2))
@@ -1121,8 +1122,8 @@ __global__ __launch_bounds__(1024) void jacobi_big_kernel(
 }
 
 // J = J0 * (product of recorded rotations), p <= 128 columns, J0 (rows x p)
-// given or the identity.  The rows of J are independent: one wave carries a row, lane k the two elements of the round's
-// pair k.  From one round-robin round to the next the first elements of the
+// given or the identity.  The rows of J are independent: one wave carries a
+// row, lane k the two elements of the round's pair k.  From one round-robin round to the next the first elements of the
 // pairs move one lane down and the second ones one lane up (the last lane
 // turns its second into a first, lane 0 its first into lane 1's second and
 // keeps the fixed column), so a round is four FMAs, one coalesced load of its
@@ -1214,7 +1215,7 @@ __global__ __launch_bounds__(64) void jacobi_accum_kernel(const double *rot,
     for (int c = lane; c < pe; c += 64)
       row[q][c] = (r0 + q < p && c == r0 + q) ? 1.0 : 0.0;
   const int ns = nsteps[0];
-  const int per = kAccChunk * npairs * 2;  // doubles per chunk (<= 2048)
+  const int per = kAccChunk * npairs * 2;  // doubles per chunk (<= 4096)
   const int64_t total = (int64_t)ns * npairs * 2;
   const int nchunks = (ns + kAccChunk - 1) / kAccChunk;
   constexpr int kPerLane = kAccChunk * (MAXD / 2) * 2 / 64;
@@ -1420,8 +1421,8 @@ void jacobi_accumulate(const double *rot, const int *nsteps, int p, double *J,
     hipLaunchKernelGGL(jacobi_replay_kernel, dim3(J0 ? rows : p), dim3(64), 0, s, rot, nsteps, p,
                        J0, J);
   } else {
-    // 2 rows per workgroup: 286 us per 128 x 128 replay against 318 us with 4
-    // rows and 394 us with 8 (D=5, chi=100)
+    // 2 rows per workgroup (timed on 128 x 128 replays, which this kernel
+    // did before jacobi_replay_kernel: 286 us, 318 us with 4 rows, 394 us with 8)
     constexpr int ROWS = 2;
     hipLaunchKernelGGL((jacobi_accum_kernel<ROWS, kMaxDimBig>), dim3(ceil_div(p, ROWS)),
                        dim3(64), 0, s, rot, nsteps, p, J);

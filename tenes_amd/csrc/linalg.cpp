@@ -258,11 +258,17 @@ SvdPending svd_top_begin_impl(Context &ctx, const Tensor *Ap, const LinearOp *op
     // second iteration on the images are nearly orthogonal columns of very
     // different lengths, which one plain pass on the scaled Gram matrix
     // orthonormalises (two for the final bases).  24 passes instead of 38 at
-    // 8 iterations; errors of the singular triplets against LAPACK unchanged
-    // over exponential, algebraic, stepped, degenerate and rank-deficient
-    // spectra of 400 x 400 matrices, and of corner spectra (D=5, chi=100,
-    // 5e-15) with 0, 1, 2, 3 or all iterations robust: 1 is taken.
-    // A warm block holds Ritz vectors and is aligned from the start.  The
+    // 8 iterations, and the same errors of the singular triplets against
+    // LAPACK over exponential, algebraic, stepped, degenerate and
+    // rank-deficient spectra of 400 x 400 matrices at 0 to 8 iterations.
+    // What is left is truncation, and depends on the Gaussian block: the
+    // subspace error is about (s_{p+1} / s_k)^(2q+1) times a constant of the
+    // block.  At D=5, chi=100 with s_129 / s_100 of 0.25 to 0.37 (to the 17th:
+    // 8e-11 to 4e-8) two blocks gave projectors 2e-12 to 3e-9 apart over 16
+    // inputs, with 38 passes as with 24.
+    // A warm block holds Ritz vectors and is taken as aligned from the start
+    // (in the first sweeps of a run, while the chi index still turns, it may
+    // miss directions that only rounding brings in).  The
     // 256-wide block keeps the shifted passes: its Ritz values reach deeper,
     // and with an environment still changing (random D=2 tensors, chi = 160,
     // 1e-2 per sweep) misaligned images lost directions to the plain pass's

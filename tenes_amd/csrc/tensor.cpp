@@ -244,8 +244,8 @@ void Context::add_lanes(int n) {
 // The runtime maps streams onto a few hardware queues (four by default) and
 // work of streams that share one runs in order: the first four side streams
 // of a process came out on two queues, so four projector chains ran two by
-// two (environment runs D=2, chi=10 / D=3, chi=27 / D=5, chi=100: 28 / 91 /
-// 252 ms; on four queues 22 / 69 / 201 ms).  Which streams share a queue
+// two (environment runs D=2, chi=10 / D=3, chi=27 / D=5, chi=100 in the order
+// of creation: 22 to 24 / 69 / 232 ms; in this order 18 / 49 / 188 ms).  Which streams share a queue
 // cannot be asked, so it is measured once per context: a short clock loop on
 // every lane, and lanes whose intervals overlap go first.  Only the order of
 // the lanes depends on it.

@@ -312,9 +312,9 @@ class Context {
   bool own_stream_ = false;
   Allocator alloc_;
   std::vector<Lane> lanes_;  // [0] = main stream, then the side streams
-  void add_lanes(int n);
-  void spread_lanes();
-  static constexpr int kLanePool = 8;  // side streams made (and ordered) at once     // creates side streams until there are n
+  void add_lanes(int n);  // creates side streams until there are n
+  void spread_lanes();    // orders them by the hardware queues they run on
+  static constexpr int kLanePool = 8;  // side streams made (and ordered) at once
   int cur_ = 0;
   int nforked_ = 0;
   int max_lanes_ = 8;
